@@ -59,30 +59,14 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "et_common.hpp"
+#include "et_gemm_common.hpp"
 
 namespace et {
 namespace {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-typedef int i32x8_t __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x8_t __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) void lds_t;
-
-// Word 3 of a gfx9 buffer descriptor for raw (untyped, stride 0) access.
-constexpr int kBufDword3 = 0x00020000;
-// A byte offset past every descriptor's num_records (all < 2^31): loads return
-// 0 and stores are dropped.
-constexpr uint32_t kOOR = 0x80000000u;
 // s_waitcnt immediate of gfx9 for lgkmcnt(0) alone (vmcnt 63, expcnt 7: no wait)
 constexpr int kWaitLgkm0 = 0xC07F;
 
-constexpr int kBM = 256;          // slots per tile
-constexpr int kBN = 256;          // output features per tile
 constexpr int kThreads = 256;
 // Slot tiles per group in the tile order: 8 for K >= 2048 (the gate/up
 // projections: 2.5-3% faster than 4 at C3 and C4), 4 below (the down
@@ -92,30 +76,13 @@ constexpr int kThreads = 256;
 constexpr int kGroupMLargeK = 8;
 constexpr int kGroupMSmallK = 4;
 constexpr int kGroupMBigExperts = 24;
+// Mean slots per expert up to which the thin kernel is considered (see
+// launch_expert_gemm).
+constexpr int64_t kThinMeanSlots = 128;
+constexpr int64_t kThinMeanSlotsWorst = 512;
 constexpr int kHalf = 256 * 128;  // one operand's chunk: 256 rows x 128 bytes
 constexpr int kStage = 2 * kHalf; // A then W; two stages fill 128 KiB of LDS
 constexpr int kSmemBytes = 2 * kStage;
-
-struct GemmArgs {
-    const unsigned char* a;         // gather: X [a_rows, K]; else A [cap, K] (bf16, or fp8 e4m3)
-    const int32_t* sorted_token;    // [cap] (gather only)
-    const unsigned char* w;         // [E, N, K] (bf16, or fp8 e4m3)
-    const int32_t* expert_offsets;  // [E + 1]
-    uint16_t* c;                    // [cap, N] bf16
-    const float* row_scale;         // [cap] (EPI_ROW_SCALE only)
-    const float* a_scale;           // fp8: [a_rows], the scale of each row of a
-    const float* w_scale;           // fp8: [E, N], the scale of each weight row
-    int64_t a_rows;
-    int64_t cap;
-    int K, N, E;                    // N: rows of each expert's weight (2 F for SwiGLU)
-};
-
-// Epilogues: the plain product; the product times a per-slot factor; or SwiGLU,
-// h = silu(g) * u of the gate rows g (weight rows 0..F-1) and the up rows u
-// (rows F..2F-1) of the same hidden unit.
-constexpr int EPI_PLAIN = ET_GEMM_PLAIN;
-constexpr int EPI_ROW_SCALE = ET_GEMM_ROW_SCALE;
-constexpr int EPI_SWIGLU = ET_GEMM_SWIGLU;
 
 // One direct-to-LDS load: this lane's 16 bytes at byte offset voff + soff of
 // the buffer land at LDS address lds + 16 * lane (soff and lds are
@@ -137,50 +104,6 @@ __device__ __forceinline__ void dma_b128(__amdgpu_buffer_rsrc_t res, uint32_t vo
 __device__ __forceinline__ void dma_b32(__amdgpu_buffer_rsrc_t res, uint32_t voff, uint32_t lds)
 {
     asm volatile("s_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(voff), "s"(res), "{m0}"(lds) : "memory");
-}
-
-// Output of one 32 x 32 accumulator tile row segment: lane l (kh = l / 32)
-// holds features 8 r + 4 kh + 0..3 of its slot in P[r] (two bf16x2 words),
-// r = 0..3.  v_permlane32_swap exchanges lanes 32..63 of its first operand
-// with lanes 0..31 of its second (lane layout checked on the device): swapping
-// P[2p] with P[2p + 1] leaves lane l with features 16 p + 8 kh + 0..7, which it
-// stores as one 16-byte write at that column (range-checked offset).
-__device__ __forceinline__ void store_row_segment(u32x2_t (&P)[4], __amdgpu_buffer_rsrc_t res, bool row_ok,
-                                                  uint32_t row_base, int col0, int ncols, int kh)
-{
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        u32x2_t& a = P[2 * p];
-        u32x2_t& b = P[2 * p + 1];
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-            const auto r = __builtin_amdgcn_permlane32_swap(a[w], b[w], false, false);
-            a[w] = r[0];
-            b[w] = r[1];
-        }
-        const int col = col0 + 16 * p + 8 * kh;
-        const u32x4_t v = {a[0], a[1], b[0], b[1]};
-        const uint32_t off = (row_ok && col < ncols) ? (row_base + (uint32_t)col) * 2u : kOOR;
-        __builtin_amdgcn_raw_buffer_store_b128(v, res, off, 0, 0);
-    }
-}
-
-// Output of two 16 x 16 accumulator tiles side by side (output columns col0
-// ... col0 + 31 of one slot): lane l (16-lane row rho = l / 16) holds columns
-// 4 rho + 0..3 of the first tile in v[0..3] and of the second in v[4..7].
-// v_permlane16_swap exchanges the odd 16-lane rows of its first operand with
-// the even rows of its second (lane layout checked on the device), after
-// which lane l holds columns 16 (rho & 1) + 8 (rho >> 1) + 0..7, stored as one
-// 16-byte write (range-checked offset; ncols is a multiple of 8).
-__device__ __forceinline__ void store_pair16(const float (&v)[8], __amdgpu_buffer_rsrc_t res, bool row_ok,
-                                             uint32_t row_base, int col0, int ncols, int rho)
-{
-    const auto lo = __builtin_amdgcn_permlane16_swap(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[4], v[5]), false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap(pack_bf16x2(v[2], v[3]), pack_bf16x2(v[6], v[7]), false, false);
-    const u32x4_t out = {lo[0], hi[0], lo[1], hi[1]};
-    const int col = col0 + 16 * (rho & 1) + 8 * (rho >> 1);
-    const uint32_t off = (row_ok && col < ncols) ? (row_base + (uint32_t)col) * 2u : kOOR;
-    __builtin_amdgcn_raw_buffer_store_b128(out, res, off, 0, 0);
 }
 
 // Wait until at most N of this wave's vector-memory operations are in flight,
@@ -205,7 +128,7 @@ __device__ __forceinline__ void dma_wait_barrier()
 // permutation of k applied to both operands (checked on the device), so the
 // fragment layouts of A and W only have to agree.
 template <bool GATHER, int EPI, bool FP8 = false>
-__global__ __launch_bounds__(kThreads) void expert_gemm_kernel(GemmArgs g)
+__global__ __launch_bounds__(kThreads) void expert_gemm_kernel(GemmArgs g, int64_t thin_rows, int cus)
 {
     constexpr int ES = FP8 ? 1 : 2;           // bytes per element
     constexpr int KC = 128 / ES;              // k per chunk (one 128-byte row)
@@ -228,6 +151,7 @@ __global__ __launch_bounds__(kThreads) void expert_gemm_kernel(GemmArgs g)
     const int E = g.E, K = g.K, N = g.N;
 
     if (wave == 0) {
+        const int64_t thin = thin_rows == 0 ? 0 : expert_gemm_split<EPI, FP8>(g, thin_rows, cus).rows;
         int carry = 0, busy = 0;
         for (int e0 = 0; e0 < E; e0 += kWave) {
             const int e = e0 + lane;
@@ -235,7 +159,7 @@ __global__ __launch_bounds__(kThreads) void expert_gemm_kernel(GemmArgs g)
             if (e < E) {
                 const int64_t lo = min<int64_t>(g.expert_offsets[e], g.cap);
                 const int64_t hi = min<int64_t>(g.expert_offsets[e + 1], g.cap);
-                n = (int)((max<int64_t>(0, hi - lo) + kBM - 1) / kBM);
+                n = hi - lo > thin ? (int)((hi - lo + kBM - 1) / kBM) : 0;
             }
             const int inc = wave_incl_scan(n) + carry;
             if (e < E) ptile[e + 1] = inc;
@@ -882,28 +806,52 @@ int launch_expert_gemm(const char* fn, int es, const void* a, int64_t a_rows, co
     const int64_t qmax = ((slot_capacity + kBM - 1) / kBM + E) * nN;
     if (qmax >= (int64_t(1) << 31))
         return fail(ET_ERR_INVALID_ARGUMENT, std::string(fn) + ": too many output tiles (slot_capacity / 256 * N / 256)");
-    const int64_t blocks = std::min<int64_t>((int64_t)num_cus(), qmax);
+    const int cus = num_cus();
+    const int64_t blocks = std::min<int64_t>((int64_t)cus, qmax);
     const dim3 grid((unsigned)(8 * ((blocks + 7) / 8)));
     hipStream_t s = static_cast<hipStream_t>(stream);
     const GemmArgs args{static_cast<const unsigned char*>(a), sorted_token, static_cast<const unsigned char*>(w),
                         expert_offsets, static_cast<uint16_t*>(c), row_scale, a_scale, w_scale, a_rows,
                         slot_capacity, (int)K, (int)N, (int)E};
     const dim3 block(kThreads);
+    // Which kernel: slot counts are on the device, so where the capacity alone
+    // does not settle it, both kernels are launched and decide there
+    // (expert_gemm_split); a launch that finds no work costs about 5 us.  Only
+    // the thin one: no expert can have more slots than one of its tiles, or
+    // even at full capacity its tiles are two rounds of one per CU at most, the
+    // time of one round of 256-row tiles.  Only the other: the capacity means
+    // more than kThinMeanSlots slots per expert, or more than
+    // kThinMeanSlotsWorst where it is a multiple of the expert count, as the
+    // capacity of a caller who has not read the slot count is (T * E, many
+    // times the routed slots).
+    const int tcols = (fp8 ? 256 : 128) / (epilogue == ET_GEMM_SWIGLU ? 2 : 1);
+    const int64_t width = epilogue == ET_GEMM_SWIGLU ? N / 2 : N;
+    const int64_t thin_max =
+        std::min<int64_t>(slot_capacity, slot_capacity / kThinTile + E) * ((width + tcols - 1) / tcols);
+    const bool only_thin =
+        slot_capacity <= kThinTile || (gather && a_rows <= kThinTile) || thin_max <= (fp8 ? 1 : 2) * (int64_t)cus;
+    const bool only_big = !only_thin &&
+                          slot_capacity > E * (slot_capacity % E == 0 ? kThinMeanSlotsWorst : kThinMeanSlots);
+    const int64_t thin_rows = only_thin ? INT64_MAX : only_big ? 0 : -1;
+    if (!only_big)
+        if (const int rc = launch_expert_gemm_thin(fp8, gather, epilogue, args, thin_rows, cus, s);
+            rc != ET_OK || only_thin)
+            return rc;
     if (fp8) {
         switch ((epilogue == ET_GEMM_SWIGLU ? 2 : 0) + (gather ? 1 : 0)) {
-            case 0: expert_gemm_kernel<false, EPI_PLAIN, true><<<grid, block, 0, s>>>(args); break;
-            case 1: expert_gemm_kernel<true, EPI_PLAIN, true><<<grid, block, 0, s>>>(args); break;
-            case 2: expert_gemm_kernel<false, EPI_SWIGLU, true><<<grid, block, 0, s>>>(args); break;
-            default: expert_gemm_kernel<true, EPI_SWIGLU, true><<<grid, block, 0, s>>>(args); break;
+            case 0: expert_gemm_kernel<false, EPI_PLAIN, true><<<grid, block, 0, s>>>(args, thin_rows, cus); break;
+            case 1: expert_gemm_kernel<true, EPI_PLAIN, true><<<grid, block, 0, s>>>(args, thin_rows, cus); break;
+            case 2: expert_gemm_kernel<false, EPI_SWIGLU, true><<<grid, block, 0, s>>>(args, thin_rows, cus); break;
+            default: expert_gemm_kernel<true, EPI_SWIGLU, true><<<grid, block, 0, s>>>(args, thin_rows, cus); break;
         }
     } else {
         switch (epilogue * 2 + (gather ? 1 : 0)) {
-            case 0: expert_gemm_kernel<false, EPI_PLAIN><<<grid, block, 0, s>>>(args); break;
-            case 1: expert_gemm_kernel<true, EPI_PLAIN><<<grid, block, 0, s>>>(args); break;
-            case 2: expert_gemm_kernel<false, EPI_ROW_SCALE><<<grid, block, 0, s>>>(args); break;
-            case 3: expert_gemm_kernel<true, EPI_ROW_SCALE><<<grid, block, 0, s>>>(args); break;
-            case 4: expert_gemm_kernel<false, EPI_SWIGLU><<<grid, block, 0, s>>>(args); break;
-            default: expert_gemm_kernel<true, EPI_SWIGLU><<<grid, block, 0, s>>>(args); break;
+            case 0: expert_gemm_kernel<false, EPI_PLAIN><<<grid, block, 0, s>>>(args, thin_rows, cus); break;
+            case 1: expert_gemm_kernel<true, EPI_PLAIN><<<grid, block, 0, s>>>(args, thin_rows, cus); break;
+            case 2: expert_gemm_kernel<false, EPI_ROW_SCALE><<<grid, block, 0, s>>>(args, thin_rows, cus); break;
+            case 3: expert_gemm_kernel<true, EPI_ROW_SCALE><<<grid, block, 0, s>>>(args, thin_rows, cus); break;
+            case 4: expert_gemm_kernel<false, EPI_SWIGLU><<<grid, block, 0, s>>>(args, thin_rows, cus); break;
+            default: expert_gemm_kernel<true, EPI_SWIGLU><<<grid, block, 0, s>>>(args, thin_rows, cus); break;
         }
     }
     return check_launch("expert_gemm_kernel");

@@ -22,7 +22,6 @@ dXp) have one row per slot.
 """
 from __future__ import annotations
 
-import ctypes
 from dataclasses import dataclass
 from typing import Optional
 
@@ -38,12 +37,29 @@ _ACT_DTYPES = {torch.float32: ET_DTYPE_F32, torch.bfloat16: ET_DTYPE_BF16}
 # helpers
 # --------------------------------------------------------------------------- #
 
+# Host cost matters here: a small call's kernels take 4 to 10 us, so a wrapper
+# that takes longer leaves the device idle.  Pointers go to ctypes as plain
+# integers, the stream handle and the current device come from torch's C
+# functions (0.1 us each; torch.cuda.current_stream() and the torch.cuda.device
+# context took 2.0 and 1.3 us of the 11 us of a one-kernel call), and an
+# argument that is fine passes one test.
+
 def _vp(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
-def _stream(device: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _call(fn: str, dev: torch.device, *args) -> None:
+    """One library call on dev's current stream (the last argument of every
+    entry point), raising on a non-zero status."""
+    f = getattr(lib(), fn)
+    index = dev.index
+    if torch._C._cuda_getDevice() == index:
+        rc = f(*args, torch._C._cuda_getCurrentRawStream(index))
+    else:
+        with torch.cuda.device(dev):
+            rc = f(*args, torch._C._cuda_getCurrentRawStream(index))
+    if rc != 0:
+        check(fn, rc)
 
 
 def _require_device(t: torch.Tensor, name: str) -> None:
@@ -54,6 +70,9 @@ def _require_device(t: torch.Tensor, name: str) -> None:
 
 
 def _require(t: torch.Tensor, name: str, dtype, ndim: int, device=None) -> None:
+    if (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == dtype and t.dim() == ndim and t.is_contiguous()
+            and (device is None or t.device == device)):
+        return
     _require_device(t, name)
     if t.dtype != dtype:
         raise TypeError(f"{name} must be {dtype}, got {t.dtype}")
@@ -72,6 +91,9 @@ def _act_dtype(t: torch.Tensor, name: str) -> int:
 
 
 def _require_act(t: torch.Tensor, name: str, device=None) -> int:
+    if (isinstance(t, torch.Tensor) and t.is_cuda and t.dim() == 2 and t.is_contiguous()
+            and (device is None or t.device == device)):
+        return _act_dtype(t, name)
     _require_device(t, name)
     dt = _act_dtype(t, name)
     if t.dim() != 2:
@@ -158,24 +180,33 @@ def route(logits: torch.Tensor, thr: torch.Tensor, *, slot_capacity: Optional[in
         workspace = torch.empty(wsb, dtype=torch.uint8, device=dev)
     elif workspace.device != dev or workspace.numel() * workspace.element_size() < wsb:
         raise ValueError(f"workspace must hold {wsb} bytes on {dev}")
-    with torch.cuda.device(dev):
-        rc = lib().et_route(_vp(logits), _vp(thr), T, E, _vp(counts), _vp(eo), _vp(to), _vp(st),
-                            _vp(sg), _vp(ts), cap, _vp(workspace), wsb, _stream(dev))
-    check("et_route", rc)
+    _call("et_route", dev, _vp(logits), _vp(thr), T, E, _vp(counts), _vp(eo), _vp(to), _vp(st), _vp(sg), _vp(ts), cap,
+          _vp(workspace), wsb)
     plan = RoutingPlan(counts, eo, to, st, sg, ts, T, E, cap)
     if sync:
         _shrink(plan, int(eo[E].item()))
     return plan
 
 
+# Slot arrays of up to this many entries stay as they were allocated.
+_KEEP_ENTRIES = 1 << 16
+
+
 def _shrink(plan: RoutingPlan, S: int) -> None:
-    """Exactly-sized copies of the slot arrays of a plan routed at capacity
-    T*E, so the T*E buffers are released (a plan held until a backward pass
-    then pins 12 bytes per slot, not per token-expert pair)."""
+    """The slot arrays of a plan routed at capacity T*E, cut to the S slots.
+    Where the capacity is large they become exactly-sized copies, so the T*E
+    buffers are released (a plan held until a backward pass then pins 12 bytes
+    per slot, not per token-expert pair); small ones (256 KiB an array at most)
+    are views, which spares a small call three copies (8 us on the device, 14
+    on the host)."""
     plan.num_slots = S
-    plan.sorted_token = plan.sorted_token[:S].clone()
-    plan.slot_gate = plan.slot_gate[:S].clone()
-    plan.token_slot = plan.token_slot[:S].clone()
+    plan.sorted_token = plan.sorted_token[:S]
+    plan.slot_gate = plan.slot_gate[:S]
+    plan.token_slot = plan.token_slot[:S]
+    if plan.capacity > _KEEP_ENTRIES:
+        plan.sorted_token = plan.sorted_token.clone()
+        plan.slot_gate = plan.slot_gate.clone()
+        plan.token_slot = plan.token_slot.clone()
     plan.capacity = S
 
 
@@ -206,10 +237,7 @@ def dispatch(x: torch.Tensor, plan: RoutingPlan, out: Optional[torch.Tensor] = N
     if T != plan.num_tokens:
         raise ValueError(f"x has {T} tokens, plan has {plan.num_tokens}")
     xp = _out_or_new(out, (plan.rows, d), x.dtype, dev, "out")
-    with torch.cuda.device(dev):
-        rc = lib().et_dispatch_fwd(_vp(x), T, d, dt, _vp(plan.token_offsets), _vp(plan.token_slot),
-                                   plan.rows, _vp(xp), _stream(dev))
-    check("et_dispatch_fwd", rc)
+    _call("et_dispatch_fwd", dev, _vp(x), T, d, dt, _vp(plan.token_offsets), _vp(plan.token_slot), plan.rows, _vp(xp))
     return xp
 
 
@@ -222,10 +250,8 @@ def combine(yp: torch.Tensor, plan: RoutingPlan, out: Optional[torch.Tensor] = N
         raise ValueError(f"yp has {yp.shape[0]} rows, plan has {plan.rows} slots")
     T, d = plan.num_tokens, yp.shape[1]
     y = _out_or_new(out, (T, d), yp.dtype, dev, "out")
-    with torch.cuda.device(dev):
-        rc = lib().et_combine_fwd(_vp(yp), _vp(plan.slot_gate), _vp(plan.token_offsets),
-                                  _vp(plan.token_slot), T, d, dt, plan.rows, _vp(y), _stream(dev))
-    check("et_combine_fwd", rc)
+    _call("et_combine_fwd", dev, _vp(yp), _vp(plan.slot_gate), _vp(plan.token_offsets), _vp(plan.token_slot), T, d,
+          dt, plan.rows, _vp(y))
     return y
 
 
@@ -267,13 +293,9 @@ def combine_backward(dy: torch.Tensor, yp: torch.Tensor, plan: RoutingPlan, *,
         workspace = torch.empty(max(wsb, 1), dtype=torch.uint8, device=dev)
     elif workspace.device != dev or workspace.numel() * workspace.element_size() < wsb:
         raise ValueError(f"workspace must hold {wsb} bytes on {dev}")
-    with torch.cuda.device(dev):
-        rc = lib().et_combine_bwd(_vp(dy), _vp(yp), _vp(plan.slot_gate), _vp(plan.sorted_token),
-                                  _vp(plan.token_offsets), _vp(plan.token_slot),
-                                  _vp(plan.expert_offsets), T, E, d, dt,
-                                  plan.rows, _vp(dyp), _vp(dgate), _vp(dl), _vp(workspace),
-                                  workspace.numel() * workspace.element_size(), _stream(dev))
-    check("et_combine_bwd", rc)
+    _call("et_combine_bwd", dev, _vp(dy), _vp(yp), _vp(plan.slot_gate), _vp(plan.sorted_token),
+          _vp(plan.token_offsets), _vp(plan.token_slot), _vp(plan.expert_offsets), T, E, d, dt, plan.rows, _vp(dyp),
+          _vp(dgate), _vp(dl), _vp(workspace), workspace.numel() * workspace.element_size())
     return dyp, dgate, dl
 
 
@@ -298,10 +320,8 @@ def dispatch_backward(dxp: torch.Tensor, plan: RoutingPlan, out: Optional[torch.
     if (router_weight is None) != (dgate is None):
         raise ValueError("router_weight and dgate go together")
     if router_weight is None:
-        with torch.cuda.device(dev):
-            rc = lib().et_dispatch_bwd(_vp(dxp), _vp(plan.token_offsets), _vp(plan.token_slot), T, d, dt,
-                                       plan.rows, _vp(dx), _stream(dev))
-        check("et_dispatch_bwd", rc)
+        _call("et_dispatch_bwd", dev, _vp(dxp), _vp(plan.token_offsets), _vp(plan.token_slot), T, d, dt, plan.rows,
+              _vp(dx))
         return dx
     E = plan.num_experts
     _require(router_weight, "router_weight", dxp.dtype, 2, dev)
@@ -315,11 +335,9 @@ def dispatch_backward(dxp: torch.Tensor, plan: RoutingPlan, out: Optional[torch.
         workspace = torch.empty(max(wsb, 1), dtype=torch.uint8, device=dev)
     elif workspace.device != dev or workspace.numel() * workspace.element_size() < wsb:
         raise ValueError(f"workspace must hold {wsb} bytes on {dev}")
-    with torch.cuda.device(dev):
-        rc = lib().et_dispatch_bwd_router(_vp(dxp), _vp(plan.token_offsets), _vp(plan.token_slot), T, d, dt,
-                                          plan.rows, _vp(plan.slot_gate), _vp(dgate), _vp(plan.expert_offsets), E,
-                                          _vp(router_weight), _vp(dx), _vp(workspace), wsb, _stream(dev))
-    check("et_dispatch_bwd_router", rc)
+    _call("et_dispatch_bwd_router", dev, _vp(dxp), _vp(plan.token_offsets), _vp(plan.token_slot), T, d, dt, plan.rows,
+          _vp(plan.slot_gate), _vp(dgate), _vp(plan.expert_offsets), E, _vp(router_weight), _vp(dx), _vp(workspace),
+          wsb)
     return dx
 
 
@@ -348,9 +366,7 @@ def router_weight_grad(dlogits: torch.Tensor, x: torch.Tensor, out: Optional[tor
         workspace = torch.empty(max(wsb, 16), dtype=torch.uint8, device=dev)
     elif workspace.device != dev or workspace.numel() * workspace.element_size() < wsb:
         raise ValueError(f"workspace must hold {wsb} bytes on {dev}")
-    with torch.cuda.device(dev):
-        rc = lib().et_router_wgrad(_vp(dlogits), _vp(x), T, d, E, _vp(dw), _vp(workspace), wsb, _stream(dev))
-    check("et_router_wgrad", rc)
+    _call("et_router_wgrad", dev, _vp(dlogits), _vp(x), T, d, E, _vp(dw), _vp(workspace), wsb)
     return dw
 
 
@@ -413,11 +429,9 @@ def expert_gemm(a: torch.Tensor, w: torch.Tensor, plan: RoutingPlan, *, gather: 
     c = _out_or_new(out, (plan.rows, ncols), torch.bfloat16, dev, "out")
     if a.data_ptr() % 16 or w.data_ptr() % 16 or c.data_ptr() % 16:
         raise ValueError("a, w and out must be 16-byte aligned")
-    with torch.cuda.device(dev):
-        rc = lib().et_expert_gemm(_vp(a), a.shape[0], _vp(plan.sorted_token) if gather else None, _vp(w),
-                                  _vp(plan.expert_offsets), E, K, N, plan.rows, _EPILOGUES[epilogue],
-                                  _vp(row_scale) if epilogue == "row_scale" else None, _vp(c), _stream(dev))
-    check("et_expert_gemm", rc)
+    _call("et_expert_gemm", dev, _vp(a), a.shape[0], _vp(plan.sorted_token) if gather else None, _vp(w),
+          _vp(plan.expert_offsets), E, K, N, plan.rows, _EPILOGUES[epilogue], _vp(row_scale) if epilogue ==
+          "row_scale" else None, _vp(c))
     return c
 
 
@@ -467,11 +481,8 @@ def expert_gemm_fp8(a: torch.Tensor, a_scale: torch.Tensor, w: torch.Tensor, w_s
         raise ValueError("a, w and out must be 16-byte aligned")
     if a_scale.data_ptr() % 4 or w_scale.data_ptr() % 4:
         raise ValueError("a_scale and w_scale must be 4-byte aligned")
-    with torch.cuda.device(dev):
-        rc = lib().et_expert_gemm_fp8(_vp(a), a.shape[0], _vp(a_scale), _vp(plan.sorted_token) if gather else None,
-                                      _vp(w), _vp(w_scale), _vp(plan.expert_offsets), E, K, N, plan.rows, epi,
-                                      _vp(c), _stream(dev))
-    check("et_expert_gemm_fp8", rc)
+    _call("et_expert_gemm_fp8", dev, _vp(a), a.shape[0], _vp(a_scale), _vp(plan.sorted_token) if gather else None,
+          _vp(w), _vp(w_scale), _vp(plan.expert_offsets), E, K, N, plan.rows, epi, _vp(c))
     return c
 
 
@@ -487,10 +498,7 @@ def expert_weight_transpose(w: torch.Tensor, plan: RoutingPlan, out: Optional[to
     if N % 8 or K % 8 or N * K >= 1 << 31:
         raise ValueError("N and K must be multiples of 8 with N * K < 2^31")
     wt = _out_or_new(out, (E, K, N), torch.bfloat16, dev, "out")
-    with torch.cuda.device(dev):
-        rc = lib().et_expert_weight_transpose(_vp(w), _vp(plan.expert_offsets), E, N, K, plan.rows, _vp(wt),
-                                              _stream(dev))
-    check("et_expert_weight_transpose", rc)
+    _call("et_expert_weight_transpose", dev, _vp(w), _vp(plan.expert_offsets), E, N, K, plan.rows, _vp(wt))
     return wt
 
 
@@ -528,10 +536,7 @@ def expert_gemm_weight_grad(dc: torch.Tensor, a: torch.Tensor, plan: RoutingPlan
     dw = _out_or_new(out, (E, N, K), torch.float32, dev, "out")
     if dc.data_ptr() % 16 or a.data_ptr() % 16:
         raise ValueError("dc and a must be 16-byte aligned")
-    with torch.cuda.device(dev):
-        rc = lib().et_expert_wgrad(_vp(dc), _vp(a), _vp(plan.expert_offsets), E, N, K, plan.rows, _vp(dw),
-                                   _stream(dev))
-    check("et_expert_wgrad", rc)
+    _call("et_expert_wgrad", dev, _vp(dc), _vp(a), _vp(plan.expert_offsets), E, N, K, plan.rows, _vp(dw))
     return dw
 
 
@@ -556,10 +561,7 @@ def swiglu(gu: torch.Tensor, plan: RoutingPlan, out: Optional[torch.Tensor] = No
     h = _out_or_new(out, (plan.rows, F), torch.bfloat16, dev, "out")
     if gu.data_ptr() % 16 or h.data_ptr() % 16:
         raise ValueError("gu and out must be 16-byte aligned")
-    with torch.cuda.device(dev):
-        rc = lib().et_swiglu_fwd(_vp(gu), F, _vp(plan.expert_offsets), plan.num_experts, plan.rows, _vp(h),
-                                 _stream(dev))
-    check("et_swiglu_fwd", rc)
+    _call("et_swiglu_fwd", dev, _vp(gu), F, _vp(plan.expert_offsets), plan.num_experts, plan.rows, _vp(h))
     return h
 
 
@@ -576,10 +578,7 @@ def swiglu_backward(gu: torch.Tensor, dh: torch.Tensor, plan: RoutingPlan,
     dgu = _out_or_new(out, (plan.rows, 2 * F), torch.bfloat16, dev, "out")
     if gu.data_ptr() % 16 or dh.data_ptr() % 16 or dgu.data_ptr() % 16:
         raise ValueError("gu, dh and out must be 16-byte aligned")
-    with torch.cuda.device(dev):
-        rc = lib().et_swiglu_bwd(_vp(gu), _vp(dh), F, _vp(plan.expert_offsets), plan.num_experts, plan.rows,
-                                 _vp(dgu), _stream(dev))
-    check("et_swiglu_bwd", rc)
+    _call("et_swiglu_bwd", dev, _vp(gu), _vp(dh), F, _vp(plan.expert_offsets), plan.num_experts, plan.rows, _vp(dgu))
     return dgu
 
 
@@ -617,10 +616,8 @@ def threshold_update_(thr: torch.Tensor, logits: torch.Tensor, k_target: int,
         workspace = torch.empty(wsb, dtype=torch.uint8, device=dev)
     elif workspace.device != dev or workspace.numel() * workspace.element_size() < wsb:
         raise ValueError(f"workspace must hold {wsb} bytes on {dev}")
-    with torch.cuda.device(dev):
-        rc = lib().et_threshold_update(_vp(logits), _vp(thr), T, E, int(k_target), float(momentum),
-                                       _vp(stat), _vp(workspace), wsb, _stream(dev))
-    check("et_threshold_update", rc)
+    _call("et_threshold_update", dev, _vp(logits), _vp(thr), T, E, int(k_target), float(momentum), _vp(stat),
+          _vp(workspace), wsb)
     return stat
 
 
@@ -671,12 +668,9 @@ def route_update(logits: torch.Tensor, thr: torch.Tensor, k_target: int, momentu
     a, b = workspace.data_ptr(), thr_workspace.data_ptr()
     if a < b + twsb and b < a + rwsb:
         raise ValueError("workspace and thr_workspace must not overlap")
-    with torch.cuda.device(dev):
-        rc = lib().et_route_update(_vp(logits), _vp(thr), T, E, _vp(counts), _vp(eo), _vp(to), _vp(st), _vp(sg),
-                                   _vp(ts), cap, _vp(workspace), rwsb, int(k_target), float(momentum),
-                                   _vp(stat) if stat is not None else None, _vp(thr_workspace), twsb,
-                                   _stream(dev))
-    check("et_route_update", rc)
+    _call("et_route_update", dev, _vp(logits), _vp(thr), T, E, _vp(counts), _vp(eo), _vp(to), _vp(st), _vp(sg),
+          _vp(ts), cap, _vp(workspace), rwsb, int(k_target), float(momentum), _vp(stat) if stat is not None else None,
+          _vp(thr_workspace), twsb)
     plan = RoutingPlan(counts, eo, to, st, sg, ts, T, E, cap)
     if sync:
         _shrink(plan, int(eo[E].item()))
@@ -709,9 +703,7 @@ def router_logits(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] 
     if x.data_ptr() % 16 or w.data_ptr() % 16:
         raise ValueError("x and w must be 16-byte aligned")
     L = _out_or_new(out, (T, E), torch.float32, dev, "out")
-    with torch.cuda.device(dev):
-        rc = lib().et_router_logits(_vp(x), _vp(w), T, d, E, _vp(L), _stream(dev))
-    check("et_router_logits", rc)
+    _call("et_router_logits", dev, _vp(x), _vp(w), T, d, E, _vp(L))
     return L
 
 
@@ -765,10 +757,8 @@ def router_route(x: torch.Tensor, w: torch.Tensor, thr: torch.Tensor, *, slot_ca
         workspace = torch.empty(wsb, dtype=torch.uint8, device=dev)
     elif workspace.device != dev or workspace.numel() * workspace.element_size() < wsb:
         raise ValueError(f"workspace must hold {wsb} bytes on {dev}")
-    with torch.cuda.device(dev):
-        rc = lib().et_router_route(_vp(x), _vp(w), _vp(thr), T, d, E, _vp(counts), _vp(eo), _vp(to), _vp(st),
-                                   _vp(sg), _vp(ts), cap, _vp(L), _vp(workspace), wsb, _stream(dev))
-    check("et_router_route", rc)
+    _call("et_router_route", dev, _vp(x), _vp(w), _vp(thr), T, d, E, _vp(counts), _vp(eo), _vp(to), _vp(st), _vp(sg),
+          _vp(ts), cap, _vp(L), _vp(workspace), wsb)
     plan = RoutingPlan(counts, eo, to, st, sg, ts, T, E, cap)
     if sync:
         _shrink(plan, int(eo[E].item()))

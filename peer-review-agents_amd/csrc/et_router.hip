@@ -482,6 +482,103 @@ __global__ __launch_bounds__(MW * kWave) void router_logits_kernel(
     }
 }
 
+// Router logits of few tokens.  The tiled kernel gives a token tile to one
+// block, which stages all of W through LDS: with a few tiles that is the time
+// of W (1 MB at 128 experts, d = 4096) through a few CUs, 35 us from 1 to 8000
+// tokens.  Here each wave owns 16 MX tokens x 16 ME experts by itself and loads
+// both operands straight into MFMA fragments (16 rows x 64 contiguous bytes a
+// load) through a register ring of U k-steps, so the same bytes stream through
+// as many CUs as there are waves, with no LDS and no barrier.  X and W are read
+// once per tile of the other, from L2.  Same k-steps in the same order as the
+// tiled kernel (v_mfma_f32_16x16x32_bf16 from k0(t) on), so the same bits.
+//
+// What bounds it is a CU's load path, about 32 GB/s whatever the ring's depth,
+// so the launch takes the smallest of the wave tiles 16 x 16, 16 x 32, 32 x 32
+// and 32 x 64 that leaves each wave a CU of its own (two waves on a CU take
+// twice as long), and the tiled kernel where none does.  Measured (us, this
+// against the tiled kernel): 128 experts, d = 4096: 8 tokens 8.0 / 34, 512 9.6 /
+// 35, 1024 13.3 / 35, 4096 24.9 / 36 (8192: 46 / 37, left to the tiled one); 64
+// experts, d = 2048: 8 tokens 5.1 / 12.6, 4096 9.7 / 13.2, 8192 14.2 / 14.0.
+constexpr int64_t kRouterSmallWaves = 256;
+
+template <int MX, int ME, int U>
+__global__ __launch_bounds__(kWave) void router_logits_small_kernel(const uint16_t* __restrict__ x,
+                                                                  const uint16_t* __restrict__ w, int T, int d, int E,
+                                                                  float* __restrict__ logits)
+{
+    const int lane = lane_id();
+    const int row = lane & 15, quad = lane >> 4;
+    const int net = (E + 16 * ME - 1) / (16 * ME);
+    const int tile = (int)blockIdx.x;
+    const int t0 = tile / net * (16 * MX), e0 = tile % net * (16 * ME);
+    if (t0 >= T) return;                                    // wave-uniform
+    const int rows = min(16 * MX, T - t0), cols = min(16 * ME, E - e0);
+    const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(x + (int64_t)t0 * d), (short)0, rows * d * 2, kBufDword3);
+    const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(w + (int64_t)e0 * d), (short)0, cols * d * 2, kBufDword3);
+    auto row_off = [&](int r, int n) -> uint32_t {          // rows past T or E read 0
+        return r < n ? (uint32_t)r * (uint32_t)d * 2u + 16u * quad : kBufOutOfRange;
+    };
+    uint32_t xo[MX], wo[ME];
+#pragma unroll
+    for (int i = 0; i < MX; ++i) xo[i] = row_off(16 * i + row, rows);
+#pragma unroll
+    for (int j = 0; j < ME; ++j) wo[j] = row_off(16 * j + row, cols);
+    const int nks = (d + 31) / 32;
+    const int first = ((t0 >> 8) & 3) * (d / 256) * 2;      // k0(t) / 32
+    const int nlim = (d - 8 * quad + 31) / 32;              // k-steps in which this lane's 8 k lie below d
+    u32x4_t xf[U][MX], wf[U][ME];
+    auto load = [&](int p, int u) {
+        const int q = min(p, nks - 1) + first;
+        const int ks = q < nks ? q : q - nks;
+        const bool in = p < nks && ks < nlim;               // (else reads 0, at a valid address)
+#pragma unroll
+        for (int i = 0; i < MX; ++i)
+            xf[u][i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                       xres, (int)(in ? xo[i] : kBufOutOfRange), ks * 64, 0));
+#pragma unroll
+        for (int j = 0; j < ME; ++j)
+            wf[u][j] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                       wres, (int)(in ? wo[j] : kBufOutOfRange), ks * 64, 0));
+    };
+    f32x4_t acc[MX][ME];
+#pragma unroll
+    for (int i = 0; i < MX; ++i)
+#pragma unroll
+        for (int j = 0; j < ME; ++j) acc[i][j] = f32x4_t{};
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        load(u, u);
+        __builtin_amdgcn_sched_barrier(0);                  // (k-step order: a wait covers the oldest only)
+    }
+    for (int p = 0; p < nks; p += U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int i = 0; i < MX; ++i)
+#pragma unroll
+                for (int j = 0; j < ME; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, xf[u][i]),
+                                                                        __builtin_bit_cast(bf16x8_t, wf[u][j]),
+                                                                        acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            load(p + u + U, u);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < MX; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int t = 16 * i + 4 * quad + r;
+#pragma unroll
+            for (int j = 0; j < ME; ++j)
+                if (t < rows && 16 * j + row < cols)
+                    logits[(int64_t)(t0 + t) * E + e0 + 16 * j + row] = acc[i][j][r];
+        }
+}
+
 // X ring length: 8-16 KiB of X in flight per wave.  The 2 x 2 launch (a
 // block of 128 tokens) keeps 4 chunks when rows are long (d >= 4096: 4-6%
 // faster there), 2 otherwise (4-7% faster at d = 1024 and 2048, where a row
@@ -563,11 +660,21 @@ extern "C" int et_router_logits(const void* x, const void* w, int64_t T, int64_t
         return fail(ET_ERR_INVALID_ARGUMENT, "et_router_logits: x and w must be 16-byte aligned");
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int nt = (int)((E + 31) / 32);
+    const uint16_t* xp = static_cast<const uint16_t*>(x);
+    const uint16_t* wp = static_cast<const uint16_t*>(w);
+    // few tokens: the smallest wave tile that leaves a CU to each wave
+    auto small = [&](auto kernel, int mx, int me) {
+        const int64_t waves = ((T + 16 * mx - 1) / (16 * mx)) * ((E + 16 * me - 1) / (16 * me));
+        if (waves > kRouterSmallWaves) return false;
+        kernel<<<dim3((unsigned)waves), dim3(kWave), 0, s>>>(xp, wp, (int)T, (int)d, (int)E, logits);
+        return true;
+    };
+    if (small(router_logits_small_kernel<1, 1, 16>, 1, 1) || small(router_logits_small_kernel<1, 2, 12>, 1, 2) ||
+        small(router_logits_small_kernel<2, 2, 8>, 2, 2) || small(router_logits_small_kernel<2, 4, 8>, 2, 4))
+        return check_launch("router_logits_small_kernel");
     const RouterLaunch L = router_launch(T);
     const int64_t ntiles = (T + 32 * L.mw * L.mt - 1) / (32 * L.mw * L.mt);
     const dim3 grid((unsigned)std::min<int64_t>(ntiles, kRouterMaxBlocks));
-    const uint16_t* xp = static_cast<const uint16_t*>(x);
-    const uint16_t* wp = static_cast<const uint16_t*>(w);
     ET_SWITCH_NT(nt, ET_SWITCH_MW(L.mw, ET_SWITCH_MT(L.mt, launch_router<NT, MW, MT, false>(
                                                                grid, s, xp, wp, T, d, E, logits, RouteEpilogue{}))));
     return check_launch("router_logits_kernel");

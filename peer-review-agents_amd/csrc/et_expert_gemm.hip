@@ -106,6 +106,19 @@ __device__ __forceinline__ void dma_b32(__amdgpu_buffer_rsrc_t res, uint32_t vof
     asm volatile("s_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(voff), "s"(res), "{m0}"(lds) : "memory");
 }
 
+// gfx950's transposing LDS read (ds_read_b64_tr_b16): within each 16-lane
+// group, if lane j points at 4 consecutive 16-bit elements M[j][0..3], lane i
+// receives M[4 m + i / 4][i % 4] for m = 0..3 (checked on the device).
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
+
+__device__ __forceinline__ uint2 read_tr16(const unsigned char* p)
+{
+    const s16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (lds_s16x4_t*)(__attribute__((address_space(3))) unsigned char*)p);
+    return __builtin_bit_cast(uint2, v);
+}
+
 // Wait until at most N of this wave's vector-memory operations are in flight,
 // then meet the other waves.  The direct-to-LDS loads count in vmcnt and are
 // in LDS once it has dropped, so after the barrier every wave's loads of the
@@ -127,7 +140,19 @@ __device__ __forceinline__ void dma_wait_barrier()
 // 16-byte segments).  The MFMA's sum over a k-step is the same for any
 // permutation of k applied to both operands (checked on the device), so the
 // fragment layouts of A and W only have to agree.
-template <bool GATHER, int EPI, bool FP8 = false>
+//
+// WT: W is [E, K, N], the sum running over its rows (the input gradient dC .
+// W_e, whose K and N are the forward's N and K).  A chunk of W is then 64 rows
+// (k) x 256 columns, loaded 2 rows x 512 contiguous bytes at a time, and the
+// fragments -- 8 consecutive k of one column per lane -- come from the
+// transposing LDS read, two to a fragment.  The 16-byte segment s of row r
+// sits at slot s ^ 4 (r & 3) ^ 2 (r / 8 & 1): the 4 rows that a 16-lane group
+// reads fall on distinct 64-byte bank windows, and the next group's on the
+// other halves of these.  Same products in the same k-steps, so the bits are
+// those of the transposed weight's product; the transpose it takes the place
+// of read and wrote every weight once more (train step at T = 65536, d = 4096,
+// E = 128, F = 1536: 2.0 ms).
+template <bool GATHER, int EPI, bool FP8 = false, bool WT = false>
 __global__ __launch_bounds__(kThreads) void expert_gemm_kernel(GemmArgs g, int64_t thin_rows, int cus)
 {
     constexpr int ES = FP8 ? 1 : 2;           // bytes per element
@@ -135,6 +160,7 @@ __global__ __launch_bounds__(kThreads) void expert_gemm_kernel(GemmArgs g, int64
     constexpr int NKS = 2;                    // k-steps per chunk (32 k bf16, 64 k fp8)
     constexpr int TS = FP8 ? 32 : 16;         // MFMA tile side
     constexpr int TM = 128 / TS;              // MFMA tiles per wave and dimension
+    static_assert(!WT || (!FP8 && EPI != EPI_SWIGLU), "transposed weights: bf16, plain or row scale");
     // the two operand stages
     __shared__ __attribute__((aligned(1024))) unsigned char smem[kSmemBytes];
     __shared__ int ptile[ET_MAX_EXPERTS + 1];    // prefix of the per-expert slot-tile counts
@@ -324,6 +350,12 @@ __global__ __launch_bounds__(kThreads) void expert_gemm_kernel(GemmArgs g, int64
         }
     };
     auto b_off = [&](const Tile& t, int i) -> uint32_t {
+        if constexpr (WT) {
+            // row r of the chunk, 8 columns at its segment
+            const int r = 16 * wave + 2 * i + (lane >> 5);
+            const int n = t.n0 + 8 * ((lane & 31) ^ (4 * (r & 3)) ^ (2 * (r >> 3 & 1)));
+            return n < N ? ((uint32_t)r * (uint32_t)N + (uint32_t)n) * 2u : kOOR;
+        }
         const int R = 64 * wave + 8 * i + (lane >> 3);
         const uint32_t seg = (uint32_t)segk[i & 1] * ES;
         if constexpr (EPI == EPI_SWIGLU) {
@@ -350,6 +382,11 @@ __global__ __launch_bounds__(kThreads) void expert_gemm_kernel(GemmArgs g, int64
         const uint32_t sb =
             lds0 + (uint32_t)((c + par) & 1) * kStage + (uint32_t)wave * 8192u + (uint32_t)i * 1024u;
         const uint32_t soff = (uint32_t)c * 128u;
+        if (WT && (q & 1)) {
+            const bool in = (c + 1) * KC <= K || c * KC + 16 * wave + 2 * i + (lane >> 5) < K;
+            dma_b128(t.wres, in ? b_off(t, i) : kOOR, soff * (uint32_t)N, sb + kHalf);
+            return;
+        }
         const uint32_t kmask = (c + 1) * KC <= K || c * KC + segk[i & 1] < K ? 0u : kOOR;
         if (q & 1) dma_b128(t.wres, b_off(t, i) | kmask, soff, sb + kHalf);
         else dma_b128(t.ares, a_off(t, o, i, tb) | kmask, soff, sb);
@@ -378,8 +415,21 @@ __global__ __launch_bounds__(kThreads) void expert_gemm_kernel(GemmArgs g, int64
     Frag f[NKS][2][TM];
     // Read r of k-step ks of the chunk in stage st, r < RPK: fragment q = r
     // (bf16) or r / 2 (fp8, piece r % 2); q < TM: A tile q, else W tile q - TM.
-    constexpr int RPK = 16;
+    // WT: the W tiles in two halves of 4 k each.
+    constexpr int RPK = WT ? 24 : 16;
+    // WT: lane l of a transposing read points at row 32 ks + 8 (l / 16) + 4
+    // half + (l % 16) / 4, columns 16 tile + 4 (l % 4) .. + 3
+    const unsigned char* const tbase =
+        smem + kHalf + (8 * rho + (r16 >> 2)) * 512 + wn * 256 + ((r16 & 3) >> 1) * 16 + (r16 & 1) * 8;
+    const int tkey = 2 * (r16 >> 2) ^ (rho & 1);
     auto read_r = [&](int st, int ks, int r) {
+        if (WT && r >= TM) {
+            const int t = (r - TM) >> 1, h = (r - TM) & 1;
+            const uint2 v = read_tr16(tbase + st * kStage + ks * 16384 + h * 2048 + ((t ^ tkey) << 5));
+            f[ks][1][t][2 * h] = v.x;
+            f[ks][1][t][2 * h + 1] = v.y;
+            return;
+        }
         const int q = FP8 ? r >> 1 : r;
         const int sgi = FP8 ? 4 * ks + 2 * (lane >> 5) + (r & 1) : 4 * ks + (lane >> 4);
         const int off = st * kStage + ((sgi ^ fkey) << 4) + (q % TM) * (TS * 128);
@@ -465,7 +515,8 @@ __global__ __launch_bounds__(kThreads) void expert_gemm_kernel(GemmArgs g, int64
             for (int m = 0; m < 32; ++m) {
                 mfma_one(0, m);
                 pin();
-                if (m & 1) read_r(st, 1, m >> 1);
+#pragma unroll
+                for (int r = m * RPK / 32; r < (m + 1) * RPK / 32; ++r) read_r(st, 1, r);
                 pin();
             }
             // (the builtin, not inline assembly: the compiler then knows these
@@ -487,7 +538,10 @@ __global__ __launch_bounds__(kThreads) void expert_gemm_kernel(GemmArgs g, int64
             for (int m = 96; m < 128; ++m) {
                 mfma_one(1, m & 63);
                 pin();
-                if (rd1 && (m & 1)) read_r(st1, 0, (m - 96) >> 1);
+                if (rd1) {
+#pragma unroll
+                    for (int r = (m - 96) * RPK / 32; r < (m - 95) * RPK / 32; ++r) read_r(st1, 0, r);
+                }
                 pin();
             }
         } else {
@@ -756,9 +810,9 @@ using namespace et;
 
 namespace {
 
-// Argument checks and launch of both entry points (es = bytes per operand
-// element: 2 for bf16, 1 for fp8).
-int launch_expert_gemm(const char* fn, int es, const void* a, int64_t a_rows, const float* a_scale,
+// Argument checks and launch of the entry points (es = bytes per operand
+// element: 2 for bf16, 1 for fp8; wt: w is [E, K, N]).
+int launch_expert_gemm(const char* fn, int es, bool wt, const void* a, int64_t a_rows, const float* a_scale,
                        const int32_t* sorted_token, const void* w, const float* w_scale,
                        const int32_t* expert_offsets, int64_t num_experts, int64_t K, int64_t N,
                        int64_t slot_capacity, int epilogue, const float* row_scale, void* c, void* stream)
@@ -829,15 +883,22 @@ int launch_expert_gemm(const char* fn, int es, const void* a, int64_t a_rows, co
     const int64_t thin_max =
         std::min<int64_t>(slot_capacity, slot_capacity / kThinTile + E) * ((width + tcols - 1) / tcols);
     const bool only_thin =
-        slot_capacity <= kThinTile || (gather && a_rows <= kThinTile) || thin_max <= (fp8 ? 1 : 2) * (int64_t)cus;
-    const bool only_big = !only_thin &&
-                          slot_capacity > E * (slot_capacity % E == 0 ? kThinMeanSlotsWorst : kThinMeanSlots);
+        !wt && (slot_capacity <= kThinTile || (gather && a_rows <= kThinTile) || thin_max <= (fp8 ? 1 : 2) * (int64_t)cus);
+    const bool only_big =
+        wt || (!only_thin && slot_capacity > E * (slot_capacity % E == 0 ? kThinMeanSlotsWorst : kThinMeanSlots));
     const int64_t thin_rows = only_thin ? INT64_MAX : only_big ? 0 : -1;
     if (!only_big)
         if (const int rc = launch_expert_gemm_thin(fp8, gather, epilogue, args, thin_rows, cus, s);
             rc != ET_OK || only_thin)
             return rc;
-    if (fp8) {
+    if (wt) {
+        switch (epilogue * 2 + (gather ? 1 : 0)) {
+            case 0: expert_gemm_kernel<false, EPI_PLAIN, false, true><<<grid, block, 0, s>>>(args, thin_rows, cus); break;
+            case 1: expert_gemm_kernel<true, EPI_PLAIN, false, true><<<grid, block, 0, s>>>(args, thin_rows, cus); break;
+            case 2: expert_gemm_kernel<false, EPI_ROW_SCALE, false, true><<<grid, block, 0, s>>>(args, thin_rows, cus); break;
+            default: expert_gemm_kernel<true, EPI_ROW_SCALE, false, true><<<grid, block, 0, s>>>(args, thin_rows, cus); break;
+        }
+    } else if (fp8) {
         switch ((epilogue == ET_GEMM_SWIGLU ? 2 : 0) + (gather ? 1 : 0)) {
             case 0: expert_gemm_kernel<false, EPI_PLAIN, true><<<grid, block, 0, s>>>(args, thin_rows, cus); break;
             case 1: expert_gemm_kernel<true, EPI_PLAIN, true><<<grid, block, 0, s>>>(args, thin_rows, cus); break;
@@ -863,8 +924,25 @@ extern "C" int et_expert_gemm(const void* a, int64_t a_rows, const int32_t* sort
                               const int32_t* expert_offsets, int64_t num_experts, int64_t K, int64_t N,
                               int64_t slot_capacity, int epilogue, const float* row_scale, void* c, void* stream)
 {
-    return launch_expert_gemm("et_expert_gemm", 2, a, a_rows, nullptr, sorted_token, w, nullptr, expert_offsets,
+    return launch_expert_gemm("et_expert_gemm", 2, false, a, a_rows, nullptr, sorted_token, w, nullptr, expert_offsets,
                               num_experts, K, N, slot_capacity, epilogue, row_scale, c, stream);
+}
+
+// The input gradient of et_expert_gemm without a transposed copy of the
+// weight: c[s, n] = the epilogue (plain, or ET_GEMM_ROW_SCALE) of sum_k
+// dc[row(s), k] * w[e(s), k, n], w bf16 [E, K, N].  Arguments otherwise as
+// et_expert_gemm's.  Not in etmoe.h: the Python API's own entry, the public C
+// form being et_expert_weight_transpose followed by et_expert_gemm.
+extern "C" int et_expert_input_grad_impl(const void* dc, int64_t dc_rows, const int32_t* sorted_token, const void* w,
+                                         const int32_t* expert_offsets, int64_t num_experts, int64_t K, int64_t N,
+                                         int64_t slot_capacity, int epilogue, const float* row_scale, void* c,
+                                         void* stream)
+{
+    const char* fn = "et_expert_input_grad_impl";
+    if (epilogue != ET_GEMM_PLAIN && epilogue != ET_GEMM_ROW_SCALE)
+        return fail(ET_ERR_INVALID_ARGUMENT, std::string(fn) + ": the input gradient has the plain and row-scale epilogues");
+    return launch_expert_gemm(fn, 2, true, dc, dc_rows, nullptr, sorted_token, w, nullptr, expert_offsets, num_experts,
+                              K, N, slot_capacity, epilogue, row_scale, c, stream);
 }
 
 extern "C" int et_expert_gemm_fp8(const void* a, int64_t a_rows, const float* a_scale, const int32_t* sorted_token,
@@ -872,7 +950,7 @@ extern "C" int et_expert_gemm_fp8(const void* a, int64_t a_rows, const float* a_
                                   int64_t num_experts, int64_t K, int64_t N, int64_t slot_capacity, int epilogue,
                                   void* c, void* stream)
 {
-    return launch_expert_gemm("et_expert_gemm_fp8", 1, a, a_rows, a_scale, sorted_token, w, w_scale, expert_offsets,
+    return launch_expert_gemm("et_expert_gemm_fp8", 1, false, a, a_rows, a_scale, sorted_token, w, w_scale, expert_offsets,
                               num_experts, K, N, slot_capacity, epilogue, nullptr, c, stream);
 }
 
@@ -983,16 +1061,6 @@ struct WgradArgs {
     int64_t cap;
     int K, N, E;
 };
-
-typedef short s16x4_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
-
-__device__ __forceinline__ uint2 read_tr16(const unsigned char* p)
-{
-    const s16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (lds_s16x4_t*)(__attribute__((address_space(3))) unsigned char*)p);
-    return __builtin_bit_cast(uint2, v);
-}
 
 __global__ __launch_bounds__(kThreads) void expert_wgrad_kernel(WgradArgs g)
 {

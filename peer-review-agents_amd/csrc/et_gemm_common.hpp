@@ -72,9 +72,10 @@ struct ThinSplit {
 // The costs compared are in 1/50 of the time of a 256-row tile and in rounds
 // of one tile per CU, as either kernel's time goes (a second thin tile on a CU
 // shares its LDS and matrix pipes).  Measured per round: bf16 (128 experts, K =
-// 4096, N = 3072) 125 us a 256-row tile, and a thin tile 53 us up to 64 slots,
-// 58 up to 96 and 62 up to 128; fp8 (64 experts, K = 2048, N = 3072) 47, and
-// 35, 37 and 39.  Calls either side of the line, thin against 256-row tiles:
+// 4096, N = 3072) 125 us a 256-row tile, and a thin tile 49 us up to 32 slots, 53
+// up to 64, 58 up to 96 and 62 up to 128, with a larger share for its start and
+// end where K is shorter (64 experts of about 64 slots, K = 1536, N = 2048: 46 and
+// 26); fp8 (64 experts, K = 2048, N = 3072) 47, and 35, 37 and 39.  Calls either side of the line, thin against 256-row tiles:
 // 128 experts of 96 slots 695 against 750 us, of 128 slots 739 against 755, of
 // 256 slots 1242 against 791; 8 experts (N = 1536) of 250 slots 57 against 81;
 // 24 experts of 128 slots (288 tiles, two rounds) 112 against 91.  Where every
@@ -88,9 +89,10 @@ __device__ __forceinline__ ThinSplit expert_gemm_split(const GemmArgs& g, int64_
     constexpr int bn = EPI == EPI_SWIGLU ? kBN / 2 : kBN, tn = kThinBlockCols<EPI, FP8>;
     const int width = EPI == EPI_SWIGLU ? g.N / 2 : g.N;
     const int64_t nb = (width + bn - 1) / bn, nt = (width + tn - 1) / tn;
-    auto cost = [](int n) -> int {   // of a tile of n slots
+    const int fixed = FP8 ? 0 : min(4, 6144 / g.K);
+    auto cost = [fixed](int n) -> int {   // of a tile of n slots
         if (n <= 0) return 0;
-        return FP8 ? (n <= 64 ? 37 : n <= 96 ? 39 : 42) : (n <= 64 ? 21 : n <= 96 ? 23 : 25);
+        return FP8 ? (n <= 64 ? 37 : n <= 96 ? 39 : 42) : fixed + (n <= 32 ? 19 : n <= 64 ? 21 : n <= 96 ? 23 : 25);
     };
     // slot tiles: thin ones and their cost, thin ones at half the height, 256-row
     // ones; and of the experts of one thin tile alone

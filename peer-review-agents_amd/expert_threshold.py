@@ -396,12 +396,19 @@ def expert_gemm(a: torch.Tensor, w: torch.Tensor, plan: RoutingPlan, *, gather: 
     ``out`` past the routed slots are left as they were.
     """
     _require(a, "a", torch.bfloat16, 2)
+    _require(w, "w", torch.bfloat16, 3, a.device)
+    _check_plan(plan, a.device)
+    E, N, K = w.shape
+    return _expert_gemm("et_expert_gemm", a, w, E, N, K, plan, gather, epilogue, row_scale, out)
+
+
+def _expert_gemm(fn: str, a, w, E: int, N: int, K: int, plan: RoutingPlan, gather: bool, epilogue: str, row_scale,
+                 out) -> torch.Tensor:
+    """The grouped GEMM of `fn` (K the length of the sum, N the product's
+    columns), its operands' dtypes and devices checked."""
     dev = a.device
-    _require(w, "w", torch.bfloat16, 3, dev)
-    _check_plan(plan, dev)
     if epilogue not in _EPILOGUES:
         raise ValueError(f"epilogue must be one of {sorted(_EPILOGUES)}, got {epilogue!r}")
-    E, N, K = w.shape
     if E != plan.num_experts:
         raise ValueError(f"w has {E} experts, plan has {plan.num_experts}")
     if a.shape[1] != K:
@@ -429,9 +436,8 @@ def expert_gemm(a: torch.Tensor, w: torch.Tensor, plan: RoutingPlan, *, gather: 
     c = _out_or_new(out, (plan.rows, ncols), torch.bfloat16, dev, "out")
     if a.data_ptr() % 16 or w.data_ptr() % 16 or c.data_ptr() % 16:
         raise ValueError("a, w and out must be 16-byte aligned")
-    _call("et_expert_gemm", dev, _vp(a), a.shape[0], _vp(plan.sorted_token) if gather else None, _vp(w),
-          _vp(plan.expert_offsets), E, K, N, plan.rows, _EPILOGUES[epilogue], _vp(row_scale) if epilogue ==
-          "row_scale" else None, _vp(c))
+    _call(fn, dev, _vp(a), a.shape[0], _vp(plan.sorted_token) if gather else None, _vp(w), _vp(plan.expert_offsets), E,
+          K, N, plan.rows, _EPILOGUES[epilogue], _vp(row_scale) if epilogue == "row_scale" else None, _vp(c))
     return c
 
 
@@ -502,21 +508,45 @@ def expert_weight_transpose(w: torch.Tensor, plan: RoutingPlan, out: Optional[to
     return wt
 
 
+def _transpose_first(E: int, N: int, K: int, rows: int) -> bool:
+    """Whether the input gradient is faster from transposed weights.  The thin
+    tiles of the grouped GEMM (few slots, or too few 256-row tiles for the chip)
+    need them: where all of a call's tiles fit at once they save 2 + 9 N / 1000
+    us of the 11 + 22 N / 1000 of a 256-row tile, and the transpose moves the
+    weights twice at 4.8 TB/s (8 experts of 262 slots, W [1536, 512]: 31 us
+    against 41 directly; [3072, 4096]: 170 against 99)."""
+    tiles = min(rows, rows // 128 + E) * -(-K // 128)
+    return tiles <= 512 and 4 * E * N * K / 4.8e6 < 2 + 9e-3 * N
+
+
 def expert_gemm_input_grad(dc: torch.Tensor, w: torch.Tensor, plan: RoutingPlan, *, gather: bool = False,
                            row_scale: Optional[torch.Tensor] = None, wt: Optional[torch.Tensor] = None,
                            out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Input gradient of :func:`expert_gemm`: da[s] = dC[row(s)] @ W[e(s)]
-    ([rows, K] bf16), through the transposed weights of the experts with slots
-    and the grouped GEMM.
+    ([rows, K] bf16), by the grouped GEMM on the weights as they are.
 
     gather=True takes dC from a token matrix [T, N] at row(s) = token(s), and
     ``row_scale`` multiplies each slot's row: with dC = dY and row_scale =
     slot_gate this is the backward of the down projection fused with the
-    combine backward (dYp = gate * dY[token] is never written).
+    combine backward (dYp = gate * dY[token] is never written).  ``wt``, a
+    [E, K, N] buffer, is filled with the transposed weights of the experts
+    with slots and the product taken from it: the same bits.
     """
-    wt = expert_weight_transpose(w, plan, out=wt)
-    return expert_gemm(dc, wt, plan, gather=gather, epilogue="row_scale" if row_scale is not None else "none",
-                       row_scale=row_scale, out=out)
+    epilogue = "row_scale" if row_scale is not None else "none"
+    _require(w, "w", torch.bfloat16, 3)
+    _check_plan(plan, w.device)
+    E, N, K = w.shape
+    if wt is not None or _transpose_first(E, N, K, plan.rows):
+        wt = expert_weight_transpose(w, plan, out=wt)
+        return expert_gemm(dc, wt, plan, gather=gather, epilogue=epilogue, row_scale=row_scale, out=out)
+    if E != plan.num_experts:
+        raise ValueError(f"w has {E} experts, plan has {plan.num_experts}")
+    if N % 8 or K % 8 or N * K >= 1 << 31:
+        raise ValueError("N and K must be multiples of 8 with N * K < 2^31")
+    _require(dc, "a", torch.bfloat16, 2)
+    if dc.device != w.device:
+        raise ValueError(f"w is on {w.device}, expected {dc.device}")
+    return _expert_gemm("et_expert_input_grad_impl", dc, w, E, K, N, plan, gather, epilogue, row_scale, out)
 
 
 def expert_gemm_weight_grad(dc: torch.Tensor, a: torch.Tensor, plan: RoutingPlan,

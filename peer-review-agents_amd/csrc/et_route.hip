@@ -1333,6 +1333,203 @@ static int pairs_place(int64_t T, int64_t E, int32_t* counts, int32_t* expert_of
     return check_launch("route_place_kernel");
 }
 
+// ---------------------------------------------------------------------------
+// Small batches: routing, and optionally the EMA update, in one block
+// ---------------------------------------------------------------------------
+
+// A small batch's three routing launches (five or six with the EMA update) take
+// 4 to 7 us each on the device and 3.5 on the host, nearly all of it launch and
+// latency.  Here one block of 16 waves does all of it: the scores go to LDS,
+// wave w takes the w-th contiguous share of the tokens (selection, counts, then
+// places, in token order), and with UPD the statistic of each expert is found
+// in its column of scores by fixing the key's bits from the top.  The rules,
+// the operations and so the bits are the other kernels'.  One CU reads the
+// logits and does every sigmoid, so it is taken for up to 256 tokens and 16384
+// scores; the statistic costs a wave 2.9 us per expert, so with the update for
+// up to 128 experts.  Measured (us on the device, this against the launches it
+// takes the place of): routing 8 tokens x 128 experts 3.6 / 13.2, 128 x 64 7.7 /
+// 11.2, 256 x 32 10.0 / 10.6, 512 x 32 17.5 / 10.6 (left to those); routing with
+// update 61 x 8 6.1 / 23, 128 x 64 19 / 24, 61 x 128 30 / 27 (and 20 us less on
+// the host), 61 x 256 58 / 38 (left to those).
+constexpr int kSmallWaves = 16;
+constexpr int kSmallThreads = kSmallWaves * kWave;
+constexpr int kSmallEntries = 16384;      // T * (E | 1) scores in LDS (64 KiB)
+constexpr int kSmallTokens = 256;
+constexpr int kSmallExperts = 256;
+constexpr int kSmallUpdateExperts = 128;
+
+struct SmallUpdate {
+    float* thr;        // [E], rewritten
+    float* stat;       // [E] or NULL
+    float m;           // momentum
+    int rank;          // c of the c-th largest score
+};
+
+// GM: expert groups of 64 (1, 2, or 4 for more than 128 experts)
+template <int GM, bool UPD>
+__global__ __launch_bounds__(kSmallThreads) void route_small_kernel(
+    const float* __restrict__ logits, const float* thr, int T, int E, int32_t* __restrict__ counts,
+    int32_t* __restrict__ expert_offsets, int32_t* __restrict__ token_offsets, int32_t* __restrict__ sorted_token,
+    float* __restrict__ slot_gate, int32_t* __restrict__ token_slot, int64_t cap, SmallUpdate up)
+{
+    __shared__ float sc[kSmallEntries];
+    __shared__ uint64_t mask[kSmallTokens * GM];    // a token's selection, by expert group
+    __shared__ int wcnt[kSmallWaves][GM * kWave];   // counts of each wave's tokens, then their bases
+    __shared__ int wslots[kSmallWaves];
+    const int tid = (int)threadIdx.x;
+    const int lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int G = (E + kWave - 1) / kWave;
+    const int P = E | 1;                             // pitch: a column's scores on distinct banks
+    float th[GM];
+    load_thresholds<GM>(thr, E, G, th);
+    for (int i = tid; i < T * E; i += kSmallThreads) {
+        const int t = i / E;
+        sc[t * P + (i - t * E)] = sigmoid(logits[i]);
+    }
+    __syncthreads();
+    // selection of the wave's tokens
+    const int per = (T + kSmallWaves - 1) / kSmallWaves;
+    const int t0 = min(wave * per, T), t1 = min(t0 + per, T);
+    int cnt[GM];
+#pragma unroll
+    for (int g = 0; g < GM; ++g) cnt[g] = 0;
+    int slots = 0;
+    for (int t = t0; t < t1; ++t) {
+        float s[GM];
+        uint64_t m[GM];
+        int k = 0;
+#pragma unroll
+        for (int g = 0; g < GM; ++g) {
+            const int e = g * kWave + lane;
+            s[g] = e < E ? sc[t * P + e] : __builtin_nanf("");
+            m[g] = (uint64_t)__ballot(s[g] >= th[g]);
+            k += (int)__popcll(m[g]);
+        }
+        if (k == 0) {
+            select_fallback<GM>(s, G, m);
+            k = 1;
+        }
+#pragma unroll
+        for (int g = 0; g < GM; ++g) {
+            cnt[g] += (int)((m[g] >> lane) & 1ull);
+            if (lane == 0) mask[t * GM + g] = m[g];
+        }
+        slots += k;
+    }
+#pragma unroll
+    for (int g = 0; g < GM; ++g) wcnt[wave][g * kWave + lane] = cnt[g];
+    if (lane == 0) wslots[wave] = slots;
+    __syncthreads();
+    if (wave == 0) {
+        // each wave's first slot per expert
+        int run = 0;
+#pragma unroll
+        for (int g = 0; g < GM; ++g) {
+            const int e = g * kWave + lane;
+            int c[kSmallWaves], tot = 0;
+#pragma unroll
+            for (int w = 0; w < kSmallWaves; ++w) {
+                c[w] = wcnt[w][e];
+                tot += c[w];
+            }
+            const int incl = wave_incl_scan(tot);
+            int at = run + incl - tot;
+            run += __builtin_amdgcn_readlane(incl, kWave - 1);
+            if (e < E) {
+                counts[e] = tot;
+                expert_offsets[e] = at;
+            }
+#pragma unroll
+            for (int w = 0; w < kSmallWaves; ++w) {
+                wcnt[w][e] = at;
+                at += c[w];
+            }
+        }
+        if (lane == 0) {
+            expert_offsets[E] = run;
+            token_offsets[T] = run;
+        }
+    }
+    __syncthreads();
+    // places of the wave's tokens
+    int base[GM];
+#pragma unroll
+    for (int g = 0; g < GM; ++g) base[g] = wcnt[wave][g * kWave + lane];
+    int pos = 0;
+    for (int w = 0; w < wave; ++w) pos += wslots[w];
+    for (int t = t0; t < t1; ++t) {
+        if (lane == 0) token_offsets[t] = pos;
+#pragma unroll
+        for (int g = 0; g < GM; ++g) {
+            const uint64_t m = mask[t * GM + g];
+            const int e = g * kWave + lane;
+            if ((m >> lane) & 1ull) {
+                const int slot = base[g]++;
+                const int entry = pos + rank_below(m);
+                if ((int64_t)entry < cap) token_slot[entry] = slot;
+                if ((int64_t)slot < cap) {
+                    sorted_token[slot] = t;
+                    slot_gate[slot] = sc[t * P + e];
+                }
+            }
+            pos += (int)__popcll(m);
+        }
+    }
+    if constexpr (UPD) {
+        // every wave read thr before the first barrier
+        constexpr int VT = kSmallTokens / kWave;
+        for (int e = wave; e < E; e += kSmallWaves) {
+            uint32_t key[VT];                        // the column's keys (NaN scores order as 0)
+#pragma unroll
+            for (int i = 0; i < VT; ++i) {
+                const int t = i * kWave + lane;
+                const float v = t < T ? sc[t * P + e] : 0.0f;
+                key[i] = v != v ? 0u : f2u(v);
+            }
+            // largest p with at least `rank` keys >= p (keys at most f2u(1) < 2^30;
+            // the zeros past T only count for p = 0, which needs no count)
+            uint32_t p = 0u;
+            for (int b = 29; b >= 0; --b) {
+                const uint32_t q = p | (1u << b);
+                int n = 0;
+#pragma unroll
+                for (int i = 0; i < VT; ++i)
+                    n += (int)__popcll((uint64_t)__ballot(key[i] >= q));
+                if (n >= up.rank) p = q;
+            }
+            if (lane == 0) {
+                const float st = u2f(p);
+                if (up.stat) up.stat[e] = st;
+                const float one_minus_m = 1.0f - up.m;
+                up.thr[e] = __builtin_fmaf(up.m, thr[e], one_minus_m * st);
+            }
+        }
+    }
+}
+
+static bool route_is_small(int64_t T, int64_t E)
+{
+    return T >= 1 && T <= kSmallTokens && E <= kSmallExperts && T * (E | 1) <= kSmallEntries;
+}
+
+template <bool UPD>
+static int launch_route_small(const float* logits, const float* thr, int64_t T, int64_t E, int32_t* counts,
+                              int32_t* expert_offsets, int32_t* token_offsets, int32_t* sorted_token,
+                              float* slot_gate, int32_t* token_slot, int64_t slot_capacity, const SmallUpdate& up,
+                              hipStream_t s)
+{
+#define ET_ROUTE_SMALL(GM_)                                                                                 \
+    route_small_kernel<GM_, UPD><<<dim3(1), dim3(kSmallThreads), 0, s>>>(                                   \
+        logits, thr, (int)T, (int)E, counts, expert_offsets, token_offsets, sorted_token, slot_gate, token_slot, \
+        slot_capacity, up)
+    if (E <= kWave) ET_ROUTE_SMALL(1);
+    else if (E <= 2 * kWave) ET_ROUTE_SMALL(2);
+    else ET_ROUTE_SMALL(4);
+#undef ET_ROUTE_SMALL
+    return check_launch("route_small_kernel");
+}
+
 // The three launches of et_route on stream s (arguments checked).
 static int route_pairs_path(const float* logits, const float* thr, int64_t T, int64_t E, int32_t* counts,
                             int32_t* expert_offsets, int32_t* token_offsets, int32_t* sorted_token,
@@ -1419,6 +1616,16 @@ int route_update_place_final(int64_t T, int64_t E, int32_t* counts, int32_t* exp
     return check_launch("route_place_kernel (with the final select)");
 }
 
+bool route_update_is_small(int64_t T, int64_t E) { return route_is_small(T, E) && E <= kSmallUpdateExperts; }
+
+int route_update_small(const float* logits, float* thr, int64_t T, int64_t E, int32_t* counts,
+                       int32_t* expert_offsets, int32_t* token_offsets, int32_t* sorted_token, float* slot_gate,
+                       int32_t* token_slot, int64_t slot_capacity, int rank, float* stat, float m, hipStream_t s)
+{
+    return launch_route_small<true>(logits, thr, T, E, counts, expert_offsets, token_offsets, sorted_token, slot_gate,
+                                    token_slot, slot_capacity, SmallUpdate{thr, stat, m, rank}, s);
+}
+
 int route_update_place(int64_t T, int64_t E, int32_t* counts, int32_t* expert_offsets, int32_t* token_offsets,
                        int32_t* sorted_token, float* slot_gate, int32_t* token_slot, int64_t slot_capacity,
                        void* workspace, hipStream_t s)
@@ -1492,6 +1699,10 @@ extern "C" int et_route(const float* logits, const float* thr, int64_t T, int64_
     if (!use_pairs(T, E))
         return route_two_read(logits, thr, T, E, counts, expert_offsets, token_offsets, sorted_token, slot_gate,
                               token_slot, slot_capacity, workspace, static_cast<hipStream_t>(stream));
+    if (route_is_small(T, E))
+        return launch_route_small<false>(logits, thr, T, E, counts, expert_offsets, token_offsets, sorted_token,
+                                         slot_gate, token_slot, slot_capacity, SmallUpdate{},
+                                         static_cast<hipStream_t>(stream));
     const PairPlan p = pair_plan(T, E);
     const PairWs ws = pair_ws_layout(workspace, p, E);
     return route_pairs_path(logits, thr, T, E, counts, expert_offsets, token_offsets, sorted_token, slot_gate,

@@ -310,6 +310,9 @@ extern "C" int et_route_update(const float* logits, float* thr, int64_t T, int64
     // select, where the route tiles hold fewer than 16 groups).
     const hipStream_t s = static_cast<hipStream_t>(stream);
     const ThrWs ws = thr_ws_layout(thr_workspace, T, E);
+    if (route_update_is_small(T, E))
+        return route_update_small(logits, thr, T, E, counts, expert_offsets, token_offsets, sorted_token, slot_gate,
+                                  token_slot, slot_capacity, (int)thr_rank(T, E, k_target), stat, momentum, s);
     if (T > 0 && E <= 4 * kWave && route_uses_pairs(T, E)) {
         const unsigned groups = (unsigned)((E + kWave - 1) / kWave);
         const dim3 grid((unsigned)ws.g.blocks, groups);

@@ -310,6 +310,11 @@ int route_update_count_bin(const float* logits, const float* thr, int64_t T, int
 int route_update_scan_collect(int64_t T, int64_t E, void* workspace, const float* logits, int nbx, int tpb,
                               const uint32_t* bin, const float* bnd, uint32_t* cand, uint32_t* cand_n,
                               hipStream_t s);
+// Small batches: routing and update in one block (et_route.hip).
+bool route_update_is_small(int64_t T, int64_t E);
+int route_update_small(const float* logits, float* thr, int64_t T, int64_t E, int32_t* counts,
+                       int32_t* expert_offsets, int32_t* token_offsets, int32_t* sorted_token, float* slot_gate,
+                       int32_t* token_slot, int64_t slot_capacity, int rank, float* stat, float m, hipStream_t s);
 int route_update_place(int64_t T, int64_t E, int32_t* counts, int32_t* expert_offsets, int32_t* token_offsets,
                        int32_t* sorted_token, float* slot_gate, int32_t* token_slot, int64_t slot_capacity,
                        void* workspace, hipStream_t s);

@@ -1805,3 +1805,56 @@ extern "C" int et_route_noalloc(const float* logits, const float* thr, int64_t T
     return route_two_read(logits, thr, T, E, counts, expert_offsets, token_offsets, sorted_token, slot_gate,
                           token_slot, slot_capacity, ws, static_cast<hipStream_t>(stream));
 }
+
+// ---------------------------------------------------------------------------
+// Exactly-sized copies of a plan's slot arrays (the Python API's own entry)
+// ---------------------------------------------------------------------------
+
+namespace et {
+namespace {
+
+struct SlotCopy {
+    const uint32_t* src[3];
+    uint32_t* dst[3];
+};
+
+// Block row y copies array y, 16 bytes per thread where both ends allow it.
+__global__ __launch_bounds__(256) void copy_slots_kernel(SlotCopy c, int64_t n, int aligned)
+{
+    const uint32_t* src = c.src[blockIdx.y];
+    uint32_t* dst = c.dst[blockIdx.y];
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (aligned && i + 4 <= n) {
+        *reinterpret_cast<uint4*>(dst + i) = *reinterpret_cast<const uint4*>(src + i);
+    } else {
+        for (int64_t j = i; j < min<int64_t>(i + 4, n); ++j) dst[j] = src[j];
+    }
+}
+
+}  // namespace
+}  // namespace et
+
+// dst = the first n entries of each of the three slot arrays, in one launch: a
+// plan routed at capacity T * E is cut to its slots once the slot count has
+// been read back, when the device is idle and three copies' launches in a row
+// are what the caller waits for (training router on 131072 tokens, 64 experts: 103 us
+// with the three copies, 93 with this).
+extern "C" int et_copy_slots_impl(const int32_t* sorted_token, const float* slot_gate, const int32_t* token_slot,
+                                  int64_t n, int32_t* sorted_token_out, float* slot_gate_out,
+                                  int32_t* token_slot_out, void* stream)
+{
+    if (n < 0 || n >= (int64_t(1) << 31)) return fail(ET_ERR_INVALID_ARGUMENT, "et_copy_slots_impl: n out of range");
+    if (n == 0) return ET_OK;
+    SlotCopy c{{reinterpret_cast<const uint32_t*>(sorted_token), reinterpret_cast<const uint32_t*>(slot_gate),
+                reinterpret_cast<const uint32_t*>(token_slot)},
+               {reinterpret_cast<uint32_t*>(sorted_token_out), reinterpret_cast<uint32_t*>(slot_gate_out),
+                reinterpret_cast<uint32_t*>(token_slot_out)}};
+    uintptr_t bits = 0;
+    for (int i = 0; i < 3; ++i) {
+        if (!c.src[i] || !c.dst[i]) return fail(ET_ERR_INVALID_ARGUMENT, "et_copy_slots_impl: null pointer");
+        bits |= reinterpret_cast<uintptr_t>(c.src[i]) | reinterpret_cast<uintptr_t>(c.dst[i]);
+    }
+    copy_slots_kernel<<<dim3((unsigned)((n + 1023) / 1024), 3), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(
+        c, n, (bits & 15) == 0);
+    return check_launch("copy_slots_kernel");
+}

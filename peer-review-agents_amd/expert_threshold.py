@@ -200,13 +200,15 @@ def _shrink(plan: RoutingPlan, S: int) -> None:
     are views, which spares a small call three copies (8 us on the device, 14
     on the host)."""
     plan.num_slots = S
-    plan.sorted_token = plan.sorted_token[:S]
-    plan.slot_gate = plan.slot_gate[:S]
-    plan.token_slot = plan.token_slot[:S]
-    if plan.capacity > _KEEP_ENTRIES:
-        plan.sorted_token = plan.sorted_token.clone()
-        plan.slot_gate = plan.slot_gate.clone()
-        plan.token_slot = plan.token_slot.clone()
+    if plan.capacity <= _KEEP_ENTRIES:
+        plan.sorted_token = plan.sorted_token[:S]
+        plan.slot_gate = plan.slot_gate[:S]
+        plan.token_slot = plan.token_slot[:S]
+    else:
+        wide = plan.sorted_token, plan.slot_gate, plan.token_slot
+        cut = tuple(torch.empty(S, dtype=t.dtype, device=t.device) for t in wide)
+        _call("et_copy_slots_impl", plan.device, *map(_vp, wide), S, *map(_vp, cut))
+        plan.sorted_token, plan.slot_gate, plan.token_slot = cut
     plan.capacity = S
 
 

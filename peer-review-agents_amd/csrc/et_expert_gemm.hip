@@ -877,15 +877,18 @@ int launch_expert_gemm(const char* fn, int es, bool wt, const void* a, int64_t a
     // more than kThinMeanSlots slots per expert, or more than
     // kThinMeanSlotsWorst where it is a multiple of the expert count, as the
     // capacity of a caller who has not read the slot count is (T * E, many
-    // times the routed slots).
+    // times the routed slots), or there are no token rows (the thin kernel's loads
+    // advance by the descriptor's scalar offset, whose range check needs one row).
     const int tcols = (fp8 ? 256 : 128) / (epilogue == ET_GEMM_SWIGLU ? 2 : 1);
     const int64_t width = epilogue == ET_GEMM_SWIGLU ? N / 2 : N;
     const int64_t thin_max =
         std::min<int64_t>(slot_capacity, slot_capacity / kThinTile + E) * ((width + tcols - 1) / tcols);
+    const bool no_thin = wt || (gather && a_rows == 0);
     const bool only_thin =
-        !wt && (slot_capacity <= kThinTile || (gather && a_rows <= kThinTile) || thin_max <= (fp8 ? 1 : 2) * (int64_t)cus);
+        !no_thin &&
+        (slot_capacity <= kThinTile || (gather && a_rows <= kThinTile) || thin_max <= (fp8 ? 1 : 2) * (int64_t)cus);
     const bool only_big =
-        wt || (!only_thin && slot_capacity > E * (slot_capacity % E == 0 ? kThinMeanSlotsWorst : kThinMeanSlots));
+        no_thin || (!only_thin && slot_capacity > E * (slot_capacity % E == 0 ? kThinMeanSlotsWorst : kThinMeanSlots));
     const int64_t thin_rows = only_thin ? INT64_MAX : only_big ? 0 : -1;
     if (!only_big)
         if (const int rc = launch_expert_gemm_thin(fp8, gather, epilogue, args, thin_rows, cus, s);

@@ -64,7 +64,8 @@ _SIGNATURES = {
     "et_router_wgrad": (_int, [_p, _p, _i64, _i64, _i64, _p, _p, _sz, _p]),
     "et_expert_gemm": (_int, [_p, _i64, _p, _p, _p, _i64, _i64, _i64, _i64, _int, _p, _p, _p]),
     "et_expert_gemm_fp8": (_int, [_p, _i64, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _int, _p, _p]),
-    # (this package's own two, not in etmoe.h)
+    # (this package's own three, not in etmoe.h)
+    "et_expert_gemm_impl": (_int, [_p, _i64, _p, _p, _p, _i64, _i64, _i64, _i64, _int, _p, _p, _i64, _p]),
     "et_copy_slots_impl": (_int, [_p, _p, _p, _i64, _p, _p, _p, _p]),
     "et_expert_input_grad_impl": (_int, [_p, _i64, _p, _p, _p, _i64, _i64, _i64, _i64, _int, _p, _p, _p]),
     "et_expert_weight_transpose": (_int, [_p, _p, _i64, _i64, _i64, _i64, _p, _p]),

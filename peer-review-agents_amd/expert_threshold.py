@@ -401,11 +401,11 @@ def expert_gemm(a: torch.Tensor, w: torch.Tensor, plan: RoutingPlan, *, gather: 
     _require(w, "w", torch.bfloat16, 3, a.device)
     _check_plan(plan, a.device)
     E, N, K = w.shape
-    return _expert_gemm("et_expert_gemm", a, w, E, N, K, plan, gather, epilogue, row_scale, out)
+    return _expert_gemm("et_expert_gemm_impl", a, w, E, N, K, plan, gather, epilogue, row_scale, out, plan.num_tokens)
 
 
 def _expert_gemm(fn: str, a, w, E: int, N: int, K: int, plan: RoutingPlan, gather: bool, epilogue: str, row_scale,
-                 out) -> torch.Tensor:
+                 out, *more: int) -> torch.Tensor:
     """The grouped GEMM of `fn` (K the length of the sum, N the product's
     columns), its operands' dtypes and devices checked."""
     dev = a.device
@@ -439,7 +439,7 @@ def _expert_gemm(fn: str, a, w, E: int, N: int, K: int, plan: RoutingPlan, gathe
     if a.data_ptr() % 16 or w.data_ptr() % 16 or c.data_ptr() % 16:
         raise ValueError("a, w and out must be 16-byte aligned")
     _call(fn, dev, _vp(a), a.shape[0], _vp(plan.sorted_token) if gather else None, _vp(w), _vp(plan.expert_offsets), E,
-          K, N, plan.rows, _EPILOGUES[epilogue], _vp(row_scale) if epilogue == "row_scale" else None, _vp(c))
+          K, N, plan.rows, _EPILOGUES[epilogue], _vp(row_scale) if epilogue == "row_scale" else None, _vp(c), *more)
     return c
 
 

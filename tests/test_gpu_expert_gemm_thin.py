@@ -116,3 +116,20 @@ def test_thin_and_256_row_tiles_give_the_same_bits(et, dev, n):
     for epilogue in ("none", "swiglu"):
         assert torch.equal(_bits(et.expert_gemm_fp8(q, sa, wq, sw, few, epilogue=epilogue)),
                            _bits(et.expert_gemm_fp8(q, sa, wq, sw, many, epilogue=epilogue)[:n]))
+
+
+@pytest.mark.parametrize("T,counts,cap", [(1, [1, 0, 1], 3), (64, [64, 0, 3] * 40, 64 * 120), (65, [65, 0, 3] * 40, 65 * 120),
+                                          (8, [300, 0, 129] * 40, 429 * 40)])
+def test_slot_major_product_of_a_small_batch(et, dev, T, counts, cap):
+    """Up to 64 tokens the thin kernel alone takes the call, above it the device
+    decides; the last plan holds more slots per expert than it names tokens."""
+    print(f"slot-major expert_gemm T={T} cap={cap}", flush=True)
+    K, N = 264, 2064
+    plan = _plan(et, dev, counts, T, T)
+    S, plan.capacity, plan.num_slots = plan.rows, cap, None
+    a = _ints((cap, K), 7, dev)
+    w = _ints((len(counts), N, K), 8, dev)
+    c = torch.full((cap, N), 7.0, device=dev, dtype=torch.bfloat16)
+    et.expert_gemm(a, w, plan, gather=False, out=c)
+    assert torch.equal(_bits(c[:S]), _bits(_reference(a, w, plan)[:S].float().to(torch.bfloat16)))
+    assert (c[S:] == 7.0).all()

@@ -64,7 +64,7 @@ _SIGNATURES = {
     "et_router_wgrad": (_int, [_p, _p, _i64, _i64, _i64, _p, _p, _sz, _p]),
     "et_expert_gemm": (_int, [_p, _i64, _p, _p, _p, _i64, _i64, _i64, _i64, _int, _p, _p, _p]),
     "et_expert_gemm_fp8": (_int, [_p, _i64, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _int, _p, _p]),
-    # (this package's own three, not in etmoe.h)
+    # (the names in _impl are this package's own, not in etmoe.h)
     "et_expert_gemm_impl": (_int, [_p, _i64, _p, _p, _p, _i64, _i64, _i64, _i64, _int, _p, _p, _i64, _p]),
     "et_copy_slots_impl": (_int, [_p, _p, _p, _i64, _p, _p, _p, _p]),
     "et_expert_input_grad_impl": (_int, [_p, _i64, _p, _p, _p, _i64, _i64, _i64, _i64, _int, _p, _p, _p]),
@@ -72,6 +72,9 @@ _SIGNATURES = {
     "et_expert_wgrad": (_int, [_p, _p, _p, _i64, _i64, _i64, _i64, _p, _p]),
     "et_swiglu_fwd": (_int, [_p, _i64, _p, _i64, _i64, _p, _p]),
     "et_swiglu_bwd": (_int, [_p, _p, _i64, _p, _i64, _i64, _p, _p]),
+    "et_swiglu_fwd_impl": (_int, [_p, _i64, _p, _i64, _i64, _p, _i64, _p]),
+    "et_swiglu_bwd_impl": (_int, [_p, _p, _i64, _p, _i64, _i64, _p, _i64, _p]),
+    "et_swiglu_blocks_impl": (_i64, [_i64, _i64, _i64, _i64]),
 }
 
 _lib = None

@@ -16,9 +16,10 @@
 // thread takes 8 hidden units of one slot (16-byte loads of g, u and dh) and
 // the slot count is read on the device, so the launch does not depend on the
 // routing (no host synchronisation).  HBM bounds them: with a block for every
-// 256 vectors (up to kMaxBlocksPerCu, which then loop) they reach 5.5 and 5.9
-// TB/s at 524288 slots of F = 1536 (0.87 and 1.36 ms; 1.08 and 1.76 ms with 8
-// looping blocks per CU and a longer sigmoid, 1.01 and 1.55 with 64 per CU).
+// 256 vectors they reach 5.9 TB/s at 524288 slots of F = 1536 (0.83 and 1.36 ms
+// forward and backward; 0.97 and 1.52 with 128 looping blocks per CU, 1.09 and
+// 1.72 with 16, whose waves drift apart and widen the range in flight).  The
+// launch, though, only knows how many slots there can be: see swiglu_blocks.
 #include <algorithm>
 
 #include "et_common.hpp"
@@ -29,8 +30,23 @@ namespace {
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
-// Bounds the blocks that find no slot where the capacity is far above the slots
+// Blocks per CU: at least where there are vectors for them, and at most.
+constexpr int64_t kMinBlocksPerCu = 16;
 constexpr int64_t kMaxBlocksPerCu = 2048;
+
+// A block for every 256 vectors of the slots that the caller knows to be there
+// (all of them after a read-back, else the batch's tokens, each of which has a
+// slot; 0 if nothing is known), the rest of the capacity by looping.  A block
+// that finds no slot costs 0.4 ns: a capacity of T * E slots, many times the
+// routed ones, took 200 us instead of 59 forward with a block for each of its
+// vectors (T = 4096, E = 128, 32768 slots of F = 1536), and takes 53 with 16 per
+// CU; 8192 slots of 524288 168 instead of 17, and 15.
+int64_t swiglu_blocks(int64_t F, int64_t slot_capacity, int64_t known_slots, int64_t cus)
+{
+    const auto blocks = [&](int64_t slots) { return (slots * (F / 8) + kThreads - 1) / kThreads; };
+    const int64_t known = std::min(blocks(std::clamp<int64_t>(known_slots, 0, slot_capacity)), cus * kMaxBlocksPerCu);
+    return std::min(blocks(slot_capacity), std::max(known, cus * kMinBlocksPerCu));
+}
 
 __device__ __forceinline__ float silu_grad_factor(float g, float s)
 {
@@ -102,7 +118,8 @@ __global__ __launch_bounds__(kThreads) void swiglu_kernel(const uint16_t* __rest
 }
 
 int launch_swiglu(const char* fn, bool bwd, const void* gu, const void* dh, int64_t F,
-                  const int32_t* expert_offsets, int64_t E, int64_t slot_capacity, void* out, void* stream)
+                  const int32_t* expert_offsets, int64_t E, int64_t slot_capacity, int64_t known_slots, void* out,
+                  void* stream)
 {
     if (E < 1 || E > ET_MAX_EXPERTS)
         return fail(ET_ERR_INVALID_ARGUMENT, std::string(fn) + ": num_experts must be in [1, " +
@@ -117,12 +134,11 @@ int launch_swiglu(const char* fn, bool bwd, const void* gu, const void* dh, int6
     if ((reinterpret_cast<uintptr_t>(gu) & 15) || (reinterpret_cast<uintptr_t>(out) & 15) ||
         (reinterpret_cast<uintptr_t>(dh) & 15))
         return fail(ET_ERR_INVALID_ARGUMENT, std::string(fn) + ": gu, dh and the output must be 16-byte aligned");
-    const int64_t vecs = slot_capacity * (F / 8);
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
-    const int64_t blocks = std::min<int64_t>((vecs + kThreads - 1) / kThreads, (int64_t)cus * kMaxBlocksPerCu);
+    const int64_t blocks = swiglu_blocks(F, slot_capacity, known_slots, cus);
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (bwd)
         swiglu_kernel<true><<<dim3((unsigned)blocks), dim3(kThreads), 0, s>>>(
@@ -143,13 +159,37 @@ using namespace et;
 extern "C" int et_swiglu_fwd(const void* gu, int64_t F, const int32_t* expert_offsets, int64_t num_experts,
                              int64_t slot_capacity, void* h, void* stream)
 {
-    return launch_swiglu("et_swiglu_fwd", false, gu, nullptr, F, expert_offsets, num_experts, slot_capacity, h,
+    return launch_swiglu("et_swiglu_fwd", false, gu, nullptr, F, expert_offsets, num_experts, slot_capacity, 0, h,
                          stream);
 }
 
 extern "C" int et_swiglu_bwd(const void* gu, const void* dh, int64_t F, const int32_t* expert_offsets,
                              int64_t num_experts, int64_t slot_capacity, void* dgu, void* stream)
 {
-    return launch_swiglu("et_swiglu_bwd", true, gu, dh, F, expert_offsets, num_experts, slot_capacity, dgu,
+    return launch_swiglu("et_swiglu_bwd", true, gu, dh, F, expert_offsets, num_experts, slot_capacity, 0, dgu,
                          stream);
+}
+
+// The Python API's own forms, not in etmoe.h: as above, for a caller who knows
+// that at least known_slots of the capacity's slots are routed.  It only sizes
+// the launch: any slot count gives the same result.
+extern "C" int et_swiglu_fwd_impl(const void* gu, int64_t F, const int32_t* expert_offsets, int64_t num_experts,
+                                  int64_t slot_capacity, void* h, int64_t known_slots, void* stream)
+{
+    return launch_swiglu("et_swiglu_fwd", false, gu, nullptr, F, expert_offsets, num_experts, slot_capacity,
+                         known_slots, h, stream);
+}
+
+extern "C" int et_swiglu_bwd_impl(const void* gu, const void* dh, int64_t F, const int32_t* expert_offsets,
+                                  int64_t num_experts, int64_t slot_capacity, void* dgu, int64_t known_slots,
+                                  void* stream)
+{
+    return launch_swiglu("et_swiglu_bwd", true, gu, dh, F, expert_offsets, num_experts, slot_capacity, known_slots,
+                         dgu, stream);
+}
+
+// Blocks of the launch on a device of `cus` compute units (for tests).
+extern "C" int64_t et_swiglu_blocks_impl(int64_t F, int64_t slot_capacity, int64_t known_slots, int64_t cus)
+{
+    return swiglu_blocks(F, slot_capacity, known_slots, cus);
 }

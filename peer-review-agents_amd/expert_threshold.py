@@ -582,6 +582,12 @@ def _swiglu_args(gu: torch.Tensor, plan: RoutingPlan) -> int:
     return gu.shape[1] // 2
 
 
+def _known_slots(plan: RoutingPlan) -> int:
+    """Slots that the host knows to be routed: all of them after a read-back,
+    else one for each token."""
+    return plan.num_slots if plan.num_slots is not None else plan.num_tokens
+
+
 def swiglu(gu: torch.Tensor, plan: RoutingPlan, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """SwiGLU of the expert FFN for training: h[s, j] = silu(g) * u with g =
     gu[s, j], u = gu[s, F + j] (gu = expert_gemm(...) without epilogue, kept for
@@ -593,7 +599,8 @@ def swiglu(gu: torch.Tensor, plan: RoutingPlan, out: Optional[torch.Tensor] = No
     h = _out_or_new(out, (plan.rows, F), torch.bfloat16, dev, "out")
     if gu.data_ptr() % 16 or h.data_ptr() % 16:
         raise ValueError("gu and out must be 16-byte aligned")
-    _call("et_swiglu_fwd", dev, _vp(gu), F, _vp(plan.expert_offsets), plan.num_experts, plan.rows, _vp(h))
+    _call("et_swiglu_fwd_impl", dev, _vp(gu), F, _vp(plan.expert_offsets), plan.num_experts, plan.rows, _vp(h),
+          _known_slots(plan))
     return h
 
 
@@ -610,7 +617,8 @@ def swiglu_backward(gu: torch.Tensor, dh: torch.Tensor, plan: RoutingPlan,
     dgu = _out_or_new(out, (plan.rows, 2 * F), torch.bfloat16, dev, "out")
     if gu.data_ptr() % 16 or dh.data_ptr() % 16 or dgu.data_ptr() % 16:
         raise ValueError("gu, dh and out must be 16-byte aligned")
-    _call("et_swiglu_bwd", dev, _vp(gu), _vp(dh), F, _vp(plan.expert_offsets), plan.num_experts, plan.rows, _vp(dgu))
+    _call("et_swiglu_bwd_impl", dev, _vp(gu), _vp(dh), F, _vp(plan.expert_offsets), plan.num_experts, plan.rows,
+          _vp(dgu), _known_slots(plan))
     return dgu
 
 

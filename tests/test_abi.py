@@ -262,3 +262,14 @@ def test_expert_gemm_fp8_rejects_bad_arguments(et):
     assert lib.et_expert_gemm_fp8(p, 16, p, p, p, p, p, 4, 64, 24, 16, 2, p, None) == ET_ERR_INVALID_ARGUMENT
     assert "SwiGLU" in _err(et)
     assert lib.et_expert_gemm_fp8(p, 16, p, p, p, p, p, 4, 64, 64, 0, 0, p, None) == 0   # nothing to do
+
+
+@pytest.mark.parametrize("F,capacity,known,blocks", [
+    (1536, 4096 * 128, 4096, 16 * 256),            # T * E slots, of which one per token is certain
+    (1536, 65536 * 128, 65536, 65536 * 192 // 256),
+    (1536, 16384 * 256, 0, 16 * 256),              # nothing known
+    (1536, 524288, 524288, 524288 * 192 // 256),   # the slot count was read back
+    (8, 1, 1, 1), (8, 300, 0, 2), (136, 1000, 1000, 67),
+    (1536, 1 << 22, 1 << 22, 2048 * 256)])
+def test_swiglu_launch_follows_the_slots_and_not_the_capacity(et, F, capacity, known, blocks):
+    assert et.lib().et_swiglu_blocks_impl(F, capacity, known, 256) == blocks

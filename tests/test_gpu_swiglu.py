@@ -112,3 +112,21 @@ def test_swiglu_rejects_bad_shapes(et, dev):
     with pytest.raises(ValueError):
         et.swiglu_backward(torch.zeros(R, 32, dtype=torch.bfloat16, device=dev),
                            torch.zeros(R, 8, dtype=torch.bfloat16, device=dev), plan)
+
+
+@pytest.mark.parametrize("T,E,F,cap", [(20000, 8, 520, 60000), (300, 64, 72, 300 * 64), (300, 64, 72, 250)])
+def test_looping_blocks_give_the_same_bits(et, dev, T, E, F, cap):
+    """A capacity not read back (16 blocks per CU, which loop) against the exact
+    slot count (a block for every 256 vectors): the first case has 1.3 million
+    vectors at least, more than the looping launch has threads."""
+    print(f"swiglu looping T={T} E={E} F={F} cap={cap}", flush=True)
+    exact, loop = _plan(et, dev, T, E, 1, seed=5), _plan(et, dev, T, E, 1, seed=5, slot_capacity=cap)
+    n = min(exact.num_slots, cap)
+    gu, dh = _random_bf16((cap, 2 * F), 1, dev), _random_bf16((cap, F), 2, dev)
+    pad = max(0, exact.num_slots - cap)
+    full = [torch.cat([t[:exact.num_slots], t[:pad]]).contiguous() for t in (gu, dh)]
+    for got, want in ((et.swiglu(gu, loop, out=torch.full_like(dh, 7.0)), et.swiglu(full[0], exact)),
+                      (et.swiglu_backward(gu, dh, loop, out=torch.full_like(gu, 7.0)),
+                       et.swiglu_backward(*full, exact))):
+        assert torch.equal(got[:n].view(torch.int16), want[:n].view(torch.int16))
+        assert bool((got[n:] == 7.0).all())

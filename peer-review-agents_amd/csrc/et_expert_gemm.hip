@@ -76,10 +76,6 @@ constexpr int kThreads = 256;
 constexpr int kGroupMLargeK = 8;
 constexpr int kGroupMSmallK = 4;
 constexpr int kGroupMBigExperts = 24;
-// Mean slots per expert up to which the thin kernel is considered (see
-// launch_expert_gemm).
-constexpr int64_t kThinMeanSlots = 128;
-constexpr int64_t kThinMeanSlotsWorst = 512;
 constexpr int kHalf = 256 * 128;  // one operand's chunk: 256 rows x 128 bytes
 constexpr int kStage = 2 * kHalf; // A then W; two stages fill 128 KiB of LDS
 constexpr int kSmemBytes = 2 * kStage;
@@ -177,7 +173,7 @@ __global__ __launch_bounds__(kThreads) void expert_gemm_kernel(GemmArgs g, int64
     const int E = g.E, K = g.K, N = g.N;
 
     if (wave == 0) {
-        const int64_t thin = thin_rows == 0 ? 0 : expert_gemm_split<EPI, FP8>(g, thin_rows, cus).rows;
+        const int64_t thin = thin_rows == 0 ? 0 : expert_gemm_split<GATHER, EPI, FP8>(g, thin_rows, cus).rows;
         int carry = 0, busy = 0;
         for (int e0 = 0; e0 < E; e0 += kWave) {
             const int e = e0 + lane;
@@ -810,14 +806,90 @@ using namespace et;
 
 namespace {
 
+// Which kernel a call goes to, from what the host knows of its slots: `capacity`
+// of them, or that many at most (!exact), an expert at most `tokens`.
+enum GemmRoute { kRouteThin = 0, kRouteBig = 1, kRouteDevice = 2 };
+
+// On the device (kRouteDevice) both kernels are launched and decide from the
+// slot counts (expert_gemm_split); the one that finds no work takes 4 to 5 us, a
+// fifth of the shortest calls.  So that is for calls of about 50 us and more and
+// for those where thin tiles may gain more than it costs; the others go to
+//   - the thin kernel where no split of the slots makes it slower: its tiles
+//     are few at their most, or no expert has more slots than one of its tiles
+//     and every count of busy experts is within 3%; also just above one round at
+//     most where a likely load has one, since a second costs 3 to 7% up to K = 2048
+//     (K = 4096, experts of up to 7/8 tile: 2 to 26%, where an idle launch costs 9);
+//   - the 256-row kernel where the mean (exact) is above a thin tile, where it may
+//     be above 512 slots per expert (the capacity T * E of more than 512 tokens),
+//     or where fp8 thin tiles lose at an even load.
+// Where the slot count is not known, a quarter of the tokens is taken as an
+// expert's likely share at most (top 8 of 32 and sparser).
+GemmRoute expert_gemm_route(const TileCall& c, int64_t E, int64_t N, int64_t capacity, bool exact, int64_t tokens)
+{
+    const int64_t width = c.swiglu ? N / 2 : N;
+    const int64_t tn = (c.fp8 ? 256 : 128) / (c.swiglu ? 2 : 1), bn = c.swiglu ? kBN / 2 : kBN;
+    const int64_t nt = (width + tn - 1) / tn, nb = (width + bn - 1) / bn;
+    // us of `tiles` 256-row tiles, from their time per round
+    const auto big_us = [&](int64_t tiles) {
+        const int64_t ns = (c.fp8 ? 12500 + 7 * (int64_t)c.K : 9300 + 167 * (int64_t)c.K / 10) + (c.swiglu ? 9000 : 0);
+        return (tiles + c.cus - 1) / c.cus * ns / 1000;
+    };
+    constexpr int64_t kDeviceUs = 50;
+    // time of `thin` thin tiles of n slots, in 1/1000 of the 256-row kernel's on
+    // `experts` of them
+    const auto ratio = [&](int64_t thin, int64_t experts, int64_t n) {
+        return 1000 * (int64_t)thin_time(c, (int)thin, thin_share(c, (int)n, (int)thin)) /
+               big_time(c, (int)(experts * nb), (int)thin);
+    };
+    const int64_t most = std::min(tokens, capacity);   // slots of one expert at most
+    const int64_t likely = exact || tokens > capacity ? most : std::max<int64_t>(1, tokens / 4);
+    if (most <= kThinTile) {
+        const int64_t all = std::min(E, capacity);
+        const auto at = [&](int64_t busy) { return ratio(busy * nt, busy, std::min(likely, (capacity + busy - 1) / busy)); };
+        int64_t lo = at(all), hi = lo;
+        for (int64_t r = 1; r <= 4; ++r)   // (both sides of each of the first rounds' ends)
+            for (int64_t busy = r * c.cus / nt; busy <= r * c.cus / nt + 1; ++busy)
+                if (busy >= 1 && busy < all) {
+                    lo = std::min(lo, at(busy));
+                    hi = std::max(hi, at(busy));
+                }
+        if (hi <= 1030) return kRouteThin;
+        if (lo >= 970) return kRouteBig;
+        if (big_us(all * nb) >= kDeviceUs) return kRouteDevice;
+        return at(all) <= 1000 ? kRouteThin : kRouteBig;
+    }
+    const int64_t mean = exact ? (capacity + E - 1) / E : std::min<int64_t>(likely, kThinTile / 2);
+    // slot tiles at most, and at a likely load
+    const int64_t tiles_max =
+        std::min(capacity / kThinTile + E, E * std::min((most + kThinTile - 1) / kThinTile, capacity)) * nt;
+    const bool spread = mean > kThinTile * 7 / 8;   // (some experts have one tile more)
+    const int64_t tiles = (spread ? mean * E / kThinTile + E / 2 : E) * nt;
+    if (thin_few(c, tiles_max)) return kRouteThin;
+    const int64_t big_min = exact ? (capacity + kBM - 1) / kBM * nb : nb;
+    if (!c.fp8 && tiles_max <= 2 * (int64_t)c.cus &&
+        thin_time(c, (int)tiles_max, thin_share(c, kThinTile, (int)tiles_max)) <= big_time(c, (int)big_min, (int)tiles_max))
+        return kRouteThin;
+    if (!c.fp8 && tiles_max <= 2 * (int64_t)c.cus && tiles <= c.cus)
+        return c.K <= 2048 || (c.K <= 4096 && !spread) ? kRouteThin : kRouteDevice;
+    if (c.fp8 && exact && tiles_max <= c.cus && thin_few(c, tiles)) return kRouteThin;
+    if (exact && mean > kThinTile) return c.fp8 && thin_few(c, tiles) ? kRouteThin : kRouteBig;
+    if (!exact && capacity > 512 * E) return kRouteBig;
+    const int64_t even = ratio(tiles, E, mean);
+    if (c.fp8 && ratio(E * nt, E, mean) > 970) return kRouteBig;
+    if (big_us(E * nb) >= kDeviceUs) return kRouteDevice;
+    // (an eighth more tiles, for an uneven load)
+    if (exact && ratio(tiles * 9 / 8, E, mean) <= 950) return kRouteThin;
+    return (1000 - even) * big_us(E * nb) >= 4500 ? kRouteDevice : kRouteBig;
+}
+
 // Argument checks and launch of the entry points (es = bytes per operand
-// element: 2 for bf16, 1 for fp8; wt: w is [E, K, N]; expert_max: slots that an
-// expert has at most, as far as the caller knows: it only picks the kernel).
+// element: 2 for bf16, 1 for fp8; wt: w is [E, K, N]; tokens, exact: see
+// expert_gemm_route, they only pick the kernel).
 int launch_expert_gemm(const char* fn, int es, bool wt, const void* a, int64_t a_rows, const float* a_scale,
                        const int32_t* sorted_token, const void* w, const float* w_scale,
                        const int32_t* expert_offsets, int64_t num_experts, int64_t K, int64_t N,
                        int64_t slot_capacity, int epilogue, const float* row_scale, void* c, void* stream,
-                       int64_t expert_max = INT64_MAX)
+                       int64_t tokens, bool exact)
 {
     const int64_t E = num_experts;
     const bool fp8 = es == 1;
@@ -870,30 +942,14 @@ int launch_expert_gemm(const char* fn, int es, bool wt, const void* a, int64_t a
                         expert_offsets, static_cast<uint16_t*>(c), row_scale, a_scale, w_scale, a_rows,
                         slot_capacity, (int)K, (int)N, (int)E};
     const dim3 block(kThreads);
-    // Which kernel: slot counts are on the device, so where the capacity alone
-    // does not settle it, both kernels are launched and decide there
-    // (expert_gemm_split); a launch that finds no work costs about 5 us.  Only
-    // the thin one: no expert can have more slots than one of its tiles, or
-    // even at full capacity its tiles are two rounds of one per CU at most, the
-    // time of one round of 256-row tiles, or the caller knows (a batch's tokens
-    // bound an expert's slots) that no expert fills more than half a tile, which
-    // takes no longer than half a 256-row tile.  Only the other: the capacity means
-    // more than kThinMeanSlots slots per expert, or more than
-    // kThinMeanSlotsWorst where it is a multiple of the expert count, as the
-    // capacity of a caller who has not read the slot count is (T * E, many
-    // times the routed slots), or there are no token rows (the thin kernel's loads
-    // advance by the descriptor's scalar offset, whose range check needs one row).
-    const int tcols = (fp8 ? 256 : 128) / (epilogue == ET_GEMM_SWIGLU ? 2 : 1);
-    const int64_t width = epilogue == ET_GEMM_SWIGLU ? N / 2 : N;
-    const int64_t thin_max =
-        std::min<int64_t>(slot_capacity, slot_capacity / kThinTile + E) * ((width + tcols - 1) / tcols);
-    const bool no_thin = wt || (gather && a_rows == 0);
-    const bool only_thin =
-        !no_thin &&
-        (slot_capacity <= kThinTile || (gather && a_rows <= kThinTile) ||
-         expert_max <= kThinTile / 2 || thin_max <= (fp8 ? 1 : 2) * (int64_t)cus);
-    const bool only_big =
-        no_thin || (!only_thin && slot_capacity > E * (slot_capacity % E == 0 ? kThinMeanSlotsWorst : kThinMeanSlots));
+    // (the transposed form has no thin tiles; nor have calls without token rows,
+    // since a thin tile's loads advance by the descriptor's scalar offset, whose
+    // range check needs one row)
+    const GemmRoute route = wt || (gather && a_rows == 0)
+                                ? kRouteBig
+                                : expert_gemm_route({(int)K, cus, fp8, epilogue == ET_GEMM_SWIGLU, gather}, E, N,
+                                                    slot_capacity, exact, gather ? std::min(tokens, a_rows) : tokens);
+    const bool only_thin = route == kRouteThin, only_big = route == kRouteBig;
     const int64_t thin_rows = only_thin ? INT64_MAX : only_big ? 0 : -1;
     if (!only_big)
         if (const int rc = launch_expert_gemm_thin(fp8, gather, epilogue, args, thin_rows, cus, s);
@@ -933,21 +989,40 @@ extern "C" int et_expert_gemm(const void* a, int64_t a_rows, const int32_t* sort
                               int64_t slot_capacity, int epilogue, const float* row_scale, void* c, void* stream)
 {
     return launch_expert_gemm("et_expert_gemm", 2, false, a, a_rows, nullptr, sorted_token, w, nullptr, expert_offsets,
-                              num_experts, K, N, slot_capacity, epilogue, row_scale, c, stream);
+                              num_experts, K, N, slot_capacity, epilogue, row_scale, c, stream, INT64_MAX, false);
 }
 
-// et_expert_gemm of a batch of num_tokens tokens, which no expert's slot count
-// exceeds: up to 64 the down projection of a batch that passes T * E as its
-// capacity is spared the 256-row launch that finds no work (whole layer forward,
-// 8 tokens on 128 experts: 377 -> 372 us; 61 on 32 experts: 439 -> 433).  Not in
-// etmoe.h: the Python API's own entry, whose plans know it.
+// et_expert_gemm and et_expert_gemm_fp8 for a caller who knows that the batch has
+// num_tokens tokens, which no expert's slot count exceeds, and whether slot_capacity
+// is the routed slot count (exact) or only holds it.  Both only pick the kernel.
+// Not in etmoe.h: the Python API's own entries, whose plans know it.
 extern "C" int et_expert_gemm_impl(const void* a, int64_t a_rows, const int32_t* sorted_token, const void* w,
                                    const int32_t* expert_offsets, int64_t num_experts, int64_t K, int64_t N,
                                    int64_t slot_capacity, int epilogue, const float* row_scale, void* c,
-                                   int64_t num_tokens, void* stream)
+                                   int64_t num_tokens, int exact, void* stream)
 {
     return launch_expert_gemm("et_expert_gemm", 2, false, a, a_rows, nullptr, sorted_token, w, nullptr, expert_offsets,
-                              num_experts, K, N, slot_capacity, epilogue, row_scale, c, stream, num_tokens);
+                              num_experts, K, N, slot_capacity, epilogue, row_scale, c, stream, num_tokens, exact != 0);
+}
+
+extern "C" int et_expert_gemm_fp8_impl(const void* a, int64_t a_rows, const float* a_scale,
+                                       const int32_t* sorted_token, const void* w, const float* w_scale,
+                                       const int32_t* expert_offsets, int64_t num_experts, int64_t K, int64_t N,
+                                       int64_t slot_capacity, int epilogue, void* c, int64_t num_tokens, int exact,
+                                       void* stream)
+{
+    return launch_expert_gemm("et_expert_gemm_fp8", 1, false, a, a_rows, a_scale, sorted_token, w, w_scale,
+                              expert_offsets, num_experts, K, N, slot_capacity, epilogue, nullptr, c, stream,
+                              num_tokens, exact != 0);
+}
+
+// The route of such a call on a device of `cus` compute units (for tests): 0 the
+// thin kernel, 1 the 256-row kernel, 2 both, deciding on the device.
+extern "C" int et_expert_gemm_route_impl(int fp8, int epilogue, int gather, int64_t num_experts, int64_t K, int64_t N,
+                                         int64_t slot_capacity, int exact, int64_t num_tokens, int cus)
+{
+    return expert_gemm_route({(int)K, cus, fp8 != 0, epilogue == ET_GEMM_SWIGLU, gather != 0}, num_experts, N,
+                             slot_capacity, exact != 0, num_tokens);
 }
 
 // The input gradient of et_expert_gemm without a transposed copy of the
@@ -964,7 +1039,7 @@ extern "C" int et_expert_input_grad_impl(const void* dc, int64_t dc_rows, const 
     if (epilogue != ET_GEMM_PLAIN && epilogue != ET_GEMM_ROW_SCALE)
         return fail(ET_ERR_INVALID_ARGUMENT, std::string(fn) + ": the input gradient has the plain and row-scale epilogues");
     return launch_expert_gemm(fn, 2, true, dc, dc_rows, nullptr, sorted_token, w, nullptr, expert_offsets, num_experts,
-                              K, N, slot_capacity, epilogue, row_scale, c, stream);
+                              K, N, slot_capacity, epilogue, row_scale, c, stream, INT64_MAX, false);
 }
 
 extern "C" int et_expert_gemm_fp8(const void* a, int64_t a_rows, const float* a_scale, const int32_t* sorted_token,
@@ -973,7 +1048,7 @@ extern "C" int et_expert_gemm_fp8(const void* a, int64_t a_rows, const float* a_
                                   void* c, void* stream)
 {
     return launch_expert_gemm("et_expert_gemm_fp8", 1, false, a, a_rows, a_scale, sorted_token, w, w_scale, expert_offsets,
-                              num_experts, K, N, slot_capacity, epilogue, nullptr, c, stream);
+                              num_experts, K, N, slot_capacity, epilogue, nullptr, c, stream, INT64_MAX, false);
 }
 
 // ---------------------------------------------------------------------------

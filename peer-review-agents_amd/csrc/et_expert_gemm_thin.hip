@@ -5,7 +5,7 @@
 // An expert with up to about a hundred slots does 2 * slots FLOP per weight
 // element, so the time is that of streaming its weight from HBM.  A 256 x 256
 // tile reads the weight through LDS with 64 KiB in flight per CU and spends
-// most of its loads, LDS writes and MFMAs on repeated rows: 4.3 TB/s on 128
+// most of its loads, LDS writes and MFMAs on repeated rows: 4.4 to 4.8 TB/s on 128
 // experts of 1 to 128 slots (K = 4096, N = 3072), and 8 experts leave half the
 // CUs idle.  Here a block of 4 waves owns the expert's slots (up to 128, in
 // MFMA tiles by their number) x 128 weight rows (fp8: 256).  A wave loads its
@@ -18,12 +18,13 @@
 // time: read from L2 by every wave instead they tripled the L2 traffic at 64
 // slots, which then bound the kernel (1.17 against 0.63 ms at 128 experts).
 //
-// Measured (us, this kernel against 256-row tiles; the weight alone takes 525
-// and 264 at 6.1 TB/s): 128 experts, K = 4096, N = 3072, of 1 slot 545 against
-// 744, of 16 551 / 736, of 64 630 / 748, of 96 695 / 750; K = 1536, N = 4096,
-// of 1 slot 301 / 372, of 64 387 / 389; 32 experts of 15 slots, K = 7168, N =
-// 3072 252 / 346; 8 experts of 8 slots, K = 4096, N = 3072 35 / 88; fp8, 64
-// experts of 32 slots, K = 2048, N = 3072 92 / 139.
+// Measured (us under sustained load, this kernel against 256-row tiles; the weight
+// alone takes 525 and 264 at 6.1 TB/s): 128 experts, K = 4096, N = 3072, of 1 slot
+// 526 against 674, of 16 570 / 679, of 64 635 / 690, of 96 697 / 704, of 128 735 /
+// 728; K = 7168, N = 1536, of 1 slot 487 / 587, of 64 589 / 601; 24 experts of 16
+// slots, K = 7168, N = 3072 240 / 286; 8 experts of 8 slots, K = 4096, N = 3072 39 /
+// 84; fp8, 64 experts of 32 slots, K = 2048, N = 3072 with SwiGLU 103 / 124.  Which
+// calls come here, and where these lose: thin_share and expert_gemm_route.
 //
 // Order of the sum: that of expert_gemm_kernel (k-steps of 32 ascending in
 // one v_mfma_f32_16x16x32_bf16 each; fp8: 64 in one
@@ -397,7 +398,7 @@ __global__ __launch_bounds__(kThreads, 2) void expert_gemm_thin_kernel(GemmArgs 
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int E = g.E;
     if (wave == 0) {
-        const ThinSplit sp = expert_gemm_split<EPI, FP8>(g, thin_rows, cus);
+        const ThinSplit sp = expert_gemm_split<GATHER, EPI, FP8>(g, thin_rows, cus);
         int carry = 0;
         for (int e0 = 0; e0 < E; e0 += kWave) {
             const int e = e0 + lane;

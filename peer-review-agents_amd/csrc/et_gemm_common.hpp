@@ -61,67 +61,141 @@ constexpr int kThinTile = 128;
 template <int EPI, bool FP8>
 constexpr int kThinBlockCols = (FP8 ? 256 : 128) / (EPI == EPI_SWIGLU ? 2 : 1);
 
+// What a call's tiles take, in 1/1000 of the time of one round (a tile per CU)
+// of 256-row tiles of the same call.  Measured over E = 8 to 128, 1 to 400 slots
+// per expert, K = 512 to 7168, N = 512 to 4096, in bursts and under sustained
+// load, plain and SwiGLU, each kernel on the whole call:
+//
+// bf16.  One round of thin tiles always wins: 0.45 to 0.55 of a round of 256-row
+// tiles up to 64 slots, 0.63 at 128 (0.9 where the weights' HBM stream binds).
+// Over many rounds a pair of thin rounds (the same weights as one of the others)
+// takes 0.83 to 0.89 of it up to 32 slots, 0.92 to 0.98 up to 64, 1.0 to 1.05 up to
+// 96, 1.01 to 1.08 up to 128: the line lies between 64 and 96, and above 128 slots
+// thin tiles lose by 20 to 100%.  Just above one round (288 tiles) the last
+// tiles run alone: K = 1024 and 2048 0.93 to 1.0 up to 64 slots, K = 4096 1.02 to
+// 1.26, K = 7168 1.08 to 1.31.
+// fp8.  Both kernels have 256 weight rows to a tile; a thin wave's load covers
+// only 32 contiguous bytes of a row, 3.3 TB/s of HBM against the 256-row tiles' 3.6
+// to 4.5.  So thin tiles win by their shorter start and end alone: K = 512 0.75 to
+// 0.95, K = 1024 0.81 to 1.02 up to 64 slots, K = 2048 0.9 to 1.0 where each has a CU
+// and 1.05 to 1.16 over many rounds, K = 4096 1.1 to 1.2, K = 7168 1.2 to 1.4 (gathered
+// rows slow the others by a tenth up to K = 1024).  With SwiGLU, whose epilogue is
+// dearer on 256 rows (9 us), 0.4 to 0.85 up to K = 2048, 0.9 to 1.0 at 4096, 1.1 to
+// 1.2 at 7168.
+struct TileCall {
+    int K, cus;
+    bool fp8, swiglu, gather;
+};
+
+// Share of a thin tile of n slots where the call has `tiles` of them.
+__host__ __device__ inline int thin_share(const TileCall& c, int n, int tiles)
+{
+    const int band = n <= 32 ? 0 : n <= 64 ? 1 : n <= 96 ? 2 : 3;
+    const auto of = [band](int a, int b, int c, int d) { return band == 0 ? a : band == 1 ? b : band == 2 ? c : d; };
+    if (n <= 0) return 0;
+    if (c.fp8) {
+        const bool light = 4 * tiles <= 3 * c.cus;   // a CU to each tile, and some to spare
+        if (c.swiglu) {
+            if (c.K <= 1024) return of(620, 680, 720, 800);
+            if (c.K <= 2048) return light ? of(700, 760, 800, 880) : of(820, 850, 870, 920);
+            if (c.K <= 4096) return light ? of(780, 840, 880, 950) : of(930, 950, 970, 1030);
+            return 1150;
+        }
+        int share = 1150;
+        if (c.K <= 512) share = light ? of(820, 880, 900, 980) : of(750, 830, 920, 1020);
+        else if (c.K <= 1024) share = light ? of(850, 900, 930, 1000) : of(900, 980, 1080, 1180);
+        else if (c.K <= 2048) share = light ? of(900, 950, 980, 1030) : of(1020, 1060, 1100, 1150);
+        else if (c.K <= 4096 && light) share = of(950, 1000, 1000, 1030);
+        return c.gather && (c.K <= 1024 || (light && c.K <= 2048)) ? share * 9 / 10 : share;
+    }
+    int share = of(445, c.K > 4096 ? 510 : 480, 515, 535);
+    if (c.swiglu) share -= share * 150 / (c.K + 150);   // (the 256-row epilogue)
+    if (c.K > 2048 && tiles > c.cus && tiles <= 3 * c.cus) share += n <= (c.K <= 4096 ? 32 : 16) ? 60 : c.K <= 4096 ? 100 : 130;
+    return share;
+}
+
+// So few thin tiles that they win whatever the slots: one round (bf16, and fp8
+// with SwiGLU up to K = 4096: 0.75 to 1.0); fp8 half a round up to K = 4096 (0.92 to
+// 1.0), with SwiGLU above that three eighths (0.85 to 0.95), half if gathered.
+__host__ __device__ inline bool thin_few(const TileCall& c, int64_t tiles)
+{
+    if (!c.fp8) return tiles <= c.cus;
+    if (c.K <= 4096) return (c.swiglu ? 1 : 2) * tiles <= c.cus;
+    return c.swiglu && 8 * tiles <= (c.gather ? 4 : 3) * c.cus;
+}
+
+// `tiles` thin tiles of this mean share.
+__host__ __device__ inline int thin_time(const TileCall& c, int tiles, int share)
+{
+    return (tiles + c.cus - 1) / c.cus * (thin_few(c, tiles) && share > 950 ? 950 : share);
+}
+
+// `tiles` 256-row tiles in a call of `thin` thin ones.  (At K = 4096 a full round
+// of bf16 weights is bound by HBM: 1.3 times a partial one's time.)
+__host__ __device__ inline int big_time(const TileCall& c, int tiles, int thin)
+{
+    const int t = (tiles + c.cus - 1) / c.cus * 1000;
+    if (c.fp8 || c.K <= 2048 || c.K > 4096 || thin > 3 * c.cus) return t;
+    const int hbm = 1300 * tiles / c.cus;
+    return t > hbm ? t : hbm;
+}
+
 // Which experts the thin kernel takes, and in tiles of how many slots.
 struct ThinSplit {
     int64_t rows;   // those with at most this many slots (0: none, INT64_MAX: all)
     int tile;       // kThinTile, or half of it
 };
 // Both kernels evaluate this on the device, where the slot counts are, with
-// one whole wave; given >= 0 is the host's answer for rows.
-//
-// The costs compared are in 1/50 of the time of a 256-row tile and in rounds
-// of one tile per CU, as either kernel's time goes (a second thin tile on a CU
-// shares its LDS and matrix pipes).  Measured per round: bf16 (128 experts, K =
-// 4096, N = 3072) 125 us a 256-row tile, and a thin tile 49 us up to 32 slots, 53
-// up to 64, 58 up to 96 and 62 up to 128, with a larger share for its start and
-// end where K is shorter (64 experts of about 64 slots, K = 1536, N = 2048: 46 and
-// 26); fp8 (64 experts, K = 2048, N = 3072) 47, and 35, 37 and 39.  Calls either side of the line, thin against 256-row tiles:
-// 128 experts of 96 slots 695 against 750 us, of 128 slots 739 against 755, of
-// 256 slots 1242 against 791; 8 experts (N = 1536) of 250 slots 57 against 81;
-// 24 experts of 128 slots (288 tiles, two rounds) 112 against 91.  Where every
-// tile of 64 slots has a CU of its own these are faster than half as many of
-// 128 (8 experts of 128 slots 38 against 54 us; of 250 slots, with more tiles
-// than CUs, 70 against 57).
-template <int EPI, bool FP8>
+// one whole wave; given >= 0 is the host's answer for rows (expert_gemm_route).
+// Where every tile of 64 slots has a CU of its own these are faster than half
+// as many of 128 (8 experts of 128 slots 38 against 54 us; of 250 slots, with more
+// tiles than CUs, 70 against 57).
+template <bool GATHER, int EPI, bool FP8>
 __device__ __forceinline__ ThinSplit expert_gemm_split(const GemmArgs& g, int64_t given, int cus)
 {
-    constexpr int kBig = 50, kHalfTile = kThinTile / 2;
-    constexpr int bn = EPI == EPI_SWIGLU ? kBN / 2 : kBN, tn = kThinBlockCols<EPI, FP8>;
-    const int width = EPI == EPI_SWIGLU ? g.N / 2 : g.N;
-    const int64_t nb = (width + bn - 1) / bn, nt = (width + tn - 1) / tn;
-    const int fixed = FP8 ? 0 : min(4, 6144 / g.K);
-    auto cost = [fixed](int n) -> int {   // of a tile of n slots
-        if (n <= 0) return 0;
-        return FP8 ? (n <= 64 ? 37 : n <= 96 ? 39 : 42) : fixed + (n <= 32 ? 19 : n <= 64 ? 21 : n <= 96 ? 23 : 25);
-    };
-    // slot tiles: thin ones and their cost, thin ones at half the height, 256-row
-    // ones; and of the experts of one thin tile alone
-    int thin = 0, thin_cost = 0, half = 0, big = 0, few = 0, few_cost = 0;
-    for (int e = lane_id(); e < g.E; e += kWave) {
+    constexpr int kHalfTile = kThinTile / 2;
+    constexpr bool swiglu = EPI == EPI_SWIGLU;
+    constexpr int bn = swiglu ? kBN / 2 : kBN, tn = kThinBlockCols<EPI, FP8>;
+    const int width = swiglu ? g.N / 2 : g.N;
+    const int nb = (width + bn - 1) / bn, nt = (width + tn - 1) / tn;
+    const auto slots = [&](int e) -> int {
         const int64_t lo = min<int64_t>(g.expert_offsets[e], g.cap);
         const int64_t hi = min<int64_t>(g.expert_offsets[e + 1], g.cap);
-        const int n = (int)max<int64_t>(0, hi - lo);
-        const int c = n / kThinTile * cost(kThinTile) + cost(n % kThinTile);
+        return (int)max<int64_t>(0, hi - lo);
+    };
+    // slot tiles: thin ones, thin ones at half the height, 256-row ones; experts of
+    // one thin tile
+    int thin = 0, half = 0, big = 0, few = 0;
+    for (int e = lane_id(); e < g.E; e += kWave) {
+        const int n = slots(e);
         thin += (n + kThinTile - 1) / kThinTile;
-        thin_cost += c;
         half += (n + kHalfTile - 1) / kHalfTile;
         big += (n + kBM - 1) / kBM;
         few += n > 0 && n <= kThinTile ? 1 : 0;
-        few_cost += n <= kThinTile ? c : 0;
     }
-    thin = wave_sum_int(thin);
-    thin_cost = wave_sum_int(thin_cost);
     half = wave_sum_int(half);
+    ThinSplit r{given, (int64_t)half * nt <= cus ? kHalfTile : kThinTile};
+    if (__builtin_expect(given >= 0, 1)) return r;
+    thin = wave_sum_int(thin);
     big = wave_sum_int(big);
     few = wave_sum_int(few);
-    few_cost = wave_sum_int(few_cost);
-    ThinSplit r{given, half * nt <= cus ? kHalfTile : kThinTile};
-    if (given >= 0) return r;
-    auto rounds = [&](int64_t tiles) { return (tiles + cus - 1) / cus; };
-    const int64_t all_thin = rounds(thin * nt) * thin_cost / max(thin, 1);
-    const int64_t all_big = rounds(big * nb) * kBig;
-    const int64_t both = rounds(few * nt) * few_cost / max(few, 1) + rounds((big - few) * nb) * kBig;
-    r.rows = all_big <= all_thin && all_big <= both ? 0 : all_thin <= both ? INT64_MAX : kThinTile;
+    // (the host sends calls of up to 512 slots per expert here: 32 bits hold these)
+    const TileCall c{g.K, cus, FP8, swiglu, GATHER};
+    int thin_shares = 0, few_shares = 0;
+    for (int e = lane_id(); e < g.E; e += kWave) {
+        const int n = slots(e);
+        if (n >= kThinTile) thin_shares += n / kThinTile * thin_share(c, kThinTile, thin * nt);
+        thin_shares += thin_share(c, n % kThinTile, thin * nt);
+        if (n <= kThinTile) few_shares += thin_share(c, n, few * nt);
+    }
+    thin_shares = wave_sum_int(thin_shares);
+    few_shares = wave_sum_int(few_shares);
+    const int all_thin = thin_time(c, thin * nt, thin_shares / max(thin, 1));
+    const int all_big = big_time(c, big * nb, thin * nt);
+    const int both = thin_time(c, few * nt, few_shares / max(few, 1)) + ((big - few) * nb + cus - 1) / cus * 1000;
+    r.rows = 20 * (int64_t)all_thin <= 19 * (int64_t)all_big && all_thin <= both ? INT64_MAX
+             : 100 * (int64_t)all_big <= 103 * (int64_t)both                     ? 0
+                                                                                 : kThinTile;
     if (r.rows == kThinTile) r.tile = kThinTile;
     return r;
 }

@@ -401,7 +401,14 @@ def expert_gemm(a: torch.Tensor, w: torch.Tensor, plan: RoutingPlan, *, gather: 
     _require(w, "w", torch.bfloat16, 3, a.device)
     _check_plan(plan, a.device)
     E, N, K = w.shape
-    return _expert_gemm("et_expert_gemm_impl", a, w, E, N, K, plan, gather, epilogue, row_scale, out, plan.num_tokens)
+    return _expert_gemm("et_expert_gemm_impl", a, w, E, N, K, plan, gather, epilogue, row_scale, out,
+                        *_known_counts(plan))
+
+
+def _known_counts(plan: RoutingPlan) -> tuple:
+    """What the host knows of the slots: an expert's at most (the tokens), and
+    whether plan.rows is their count."""
+    return plan.num_tokens, int(plan.num_slots is not None)
 
 
 def _expert_gemm(fn: str, a, w, E: int, N: int, K: int, plan: RoutingPlan, gather: bool, epilogue: str, row_scale,
@@ -489,8 +496,8 @@ def expert_gemm_fp8(a: torch.Tensor, a_scale: torch.Tensor, w: torch.Tensor, w_s
         raise ValueError("a, w and out must be 16-byte aligned")
     if a_scale.data_ptr() % 4 or w_scale.data_ptr() % 4:
         raise ValueError("a_scale and w_scale must be 4-byte aligned")
-    _call("et_expert_gemm_fp8", dev, _vp(a), a.shape[0], _vp(a_scale), _vp(plan.sorted_token) if gather else None,
-          _vp(w), _vp(w_scale), _vp(plan.expert_offsets), E, K, N, plan.rows, epi, _vp(c))
+    _call("et_expert_gemm_fp8_impl", dev, _vp(a), a.shape[0], _vp(a_scale), _vp(plan.sorted_token) if gather else None,
+          _vp(w), _vp(w_scale), _vp(plan.expert_offsets), E, K, N, plan.rows, epi, _vp(c), *_known_counts(plan))
     return c
 
 

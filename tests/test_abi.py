@@ -273,3 +273,51 @@ def test_expert_gemm_fp8_rejects_bad_arguments(et):
     (1536, 1 << 22, 1 << 22, 2048 * 256)])
 def test_swiglu_launch_follows_the_slots_and_not_the_capacity(et, F, capacity, known, blocks):
     assert et.lib().et_swiglu_blocks_impl(F, capacity, known, 256) == blocks
+
+
+THIN, BIG, DEVICE = 0, 1, 2
+MANY = 1 << 62      # no bound on an expert's slots
+
+
+@pytest.mark.parametrize("fp8,epilogue,gather,E,K,N,capacity,exact,tokens,routes", [
+    # one to two rounds of thin tiles, not the thin kernel unseen (us, thin / 256-row): 205 / 162
+    (0, 0, 0, 24, 7168, 1536, 24 * 96, 1, MANY, (BIG, DEVICE)),
+    (0, 0, 0, 8, 4096, 1536, 8 * 512, 1, MANY, (BIG,)),             # 87 / 84
+    (0, 0, 0, 1, 7168, 3072, 2048, 1, MANY, (BIG,)),                # 152 / 138
+    (0, 0, 0, 12, 7168, 1536, 12 * 256, 1, MANY, (BIG, DEVICE)),    # 181 / 166
+    # one round at most: 17 / 24, 85 / 154; at a likely load and a short sum: 40 / 40
+    (0, 0, 0, 8, 512, 512, 8 * 262, 1, MANY, (THIN,)),
+    (0, 0, 0, 8, 7168, 512, 8 * 262, 1, MANY, (THIN,)),
+    (0, 0, 0, 8, 1536, 1536, 8 * 250, 1, MANY, (THIN,)),
+    # fp8 streams weights slower through thin tiles: 78 / 67, 212 / 150, 71 / 55
+    (1, 0, 0, 32, 7168, 1024, 32 * 64, 1, MANY, (BIG,)),
+    (1, 0, 0, 24, 7168, 3072, 24 * 64, 1, MANY, (BIG,)),
+    (1, 0, 0, 64, 2048, 1536, 64 * 128, 1, MANY, (BIG,)),
+    (1, 2, 1, 24, 7168, 512, 24 * 64, 1, MANY, (THIN,)),            # 65 / 78 with SwiGLU
+    # short calls do not pay for a launch that finds no work: 22 and 26 us of 256-row tiles
+    (0, 0, 0, 24, 512, 1536, 24 * 128, 1, MANY, (BIG,)),
+    (0, 0, 0, 128, 512, 512, 128 * 96, 1, MANY, (BIG,)),
+    # decode batches at the capacity T * E: gate/up and down projection
+    (0, 2, 1, 128, 4096, 3072, 8 * 128, 0, 8, (THIN,)),
+    (0, 0, 0, 128, 1536, 4096, 8 * 128, 0, 8, (THIN,)),
+    (0, 2, 1, 32, 7168, 3072, 61 * 32, 0, 61, (THIN,)),
+    (0, 0, 0, 32, 1536, 7168, 61 * 32, 0, 61, (THIN,)),
+    # light experts, some perhaps heavy: the device sees
+    (0, 0, 0, 128, 4096, 3072, 128 * 30, 1, 4000, (DEVICE,)),
+    (0, 2, 1, 128, 4096, 3072, 512 * 128, 0, 512, (DEVICE,)),
+    (0, 2, 1, 128, 4096, 3072, 600 * 128, 0, 600, (BIG,)),
+    # prefill and training
+    (0, 2, 1, 128, 4096, 3072, 24008, 1, 3001, (BIG,)),
+    (0, 0, 0, 64, 1536, 2048, 131072, 1, 16384, (BIG,))])
+def test_expert_gemm_route(et, fp8, epilogue, gather, E, K, N, capacity, exact, tokens, routes):
+    assert et.lib().et_expert_gemm_route_impl(fp8, epilogue, gather, E, K, N, capacity, exact, tokens, 256) in routes
+
+
+def test_expert_gemm_route_does_not_read_the_capacitys_divisors(et):
+    """A slot count that happens to be a multiple of the expert count is a slot
+    count like its neighbours."""
+    def route(S, exact):
+        return et.lib().et_expert_gemm_route_impl(0, 0, 0, 64, 2048, 1536, S, exact, MANY, 256)
+    for mean in (40, 100, 200, 300, 500, 600):
+        for exact in (0, 1):
+            assert route(64 * mean - 1, exact) == route(64 * mean, exact), (mean, exact)

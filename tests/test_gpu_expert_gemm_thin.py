@@ -133,3 +133,34 @@ def test_slot_major_product_of_a_small_batch(et, dev, T, counts, cap):
     et.expert_gemm(a, w, plan, gather=False, out=c)
     assert torch.equal(_bits(c[:S]), _bits(_reference(a, w, plan)[:S].float().to(torch.bfloat16)))
     assert (c[S:] == 7.0).all()
+
+
+@pytest.mark.parametrize("counts", [[20] * 40, [390, 400, 0, 410] * 10, [2000] + [20] * 9 + [1] * 10 + [2000] + [129] * 9 + [0] * 10])
+def test_device_decides_from_the_slot_counts(et, dev, counts):
+    """A slot count that was not read back: both kernels are launched, and light
+    experts, heavy ones or each take the one or the other; the same rows as of
+    the exact plan."""
+    E, T, K, N, S = len(counts), 4000, 1040, 3072, sum(counts)
+    print(f"expert_gemm decided on the device S={S}", flush=True)
+    exact = _plan(et, dev, counts, T, 11)
+    cap = S + 7
+    pad = torch.zeros(7, dtype=torch.int32, device=dev)
+    plan = et.RoutingPlan(exact.counts, exact.expert_offsets, exact.token_offsets, torch.cat([exact.sorted_token, pad]),
+                          torch.cat([exact.slot_gate, pad.float()]), exact.token_slot, T, E, cap)
+    for fp8, epi in ((0, 0), (0, 2)):
+        assert et.lib().et_expert_gemm_route_impl(fp8, epi, 1, E, K, N, cap, 0, T, 256) == 2
+    x, w = _ints((T, K), 12, dev), _ints((E, N, K), 13, dev)
+    want = _bits(_reference(x[exact.sorted_token.long()], w, exact).float().to(torch.bfloat16))
+    xp = torch.cat([x[exact.sorted_token.long()], x[:7]]).contiguous()
+    for gather, a in ((True, x), (False, xp)):
+        c = torch.full((cap, N), 7.0, device=dev, dtype=torch.bfloat16)
+        et.expert_gemm(a, w, plan, gather=gather, out=c)
+        assert torch.equal(_bits(c[:S]), want) and bool((c[S:] == 7.0).all())
+        h = et.expert_gemm(a, w, plan, gather=gather, epilogue="swiglu")
+        assert torch.equal(_bits(h[:S]), _bits(et.expert_gemm(a[:S] if not gather else a, w, exact, gather=gather,
+                                                              epilogue="swiglu")))
+    q, wq = x.to(F8), w.to(F8)
+    sa, sw = torch.ones(T, device=dev), torch.ones(E, N, device=dev)
+    for epilogue in ("none", "swiglu"):
+        assert torch.equal(_bits(et.expert_gemm_fp8(q, sa, wq, sw, plan, epilogue=epilogue)[:S]),
+                           _bits(et.expert_gemm_fp8(q, sa, wq, sw, exact, epilogue=epilogue)))

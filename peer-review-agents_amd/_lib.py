@@ -69,6 +69,7 @@ _SIGNATURES = {
     "et_expert_gemm_fp8_impl": (_int, [_p, _i64, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _int, _p, _i64, _int,
                                        _p]),
     "et_expert_gemm_route_impl": (_int, [_int, _int, _int, _i64, _i64, _i64, _i64, _int, _i64, _int]),
+    "et_expert_input_grad_transposes_impl": (_int, [_i64, _i64, _i64, _i64, _i64, _int]),
     "et_copy_slots_impl": (_int, [_p, _p, _p, _i64, _p, _p, _p, _p]),
     "et_expert_input_grad_impl": (_int, [_p, _i64, _p, _p, _p, _i64, _i64, _i64, _i64, _int, _p, _p, _p]),
     "et_expert_weight_transpose": (_int, [_p, _p, _i64, _i64, _i64, _i64, _p, _p]),

@@ -517,15 +517,10 @@ def expert_weight_transpose(w: torch.Tensor, plan: RoutingPlan, out: Optional[to
     return wt
 
 
-def _transpose_first(E: int, N: int, K: int, rows: int) -> bool:
-    """Whether the input gradient is faster from transposed weights.  The thin
-    tiles of the grouped GEMM (few slots, or too few 256-row tiles for the chip)
-    need them: where all of a call's tiles fit at once they save 2 + 9 N / 1000
-    us of the 11 + 22 N / 1000 of a 256-row tile, and the transpose moves the
-    weights twice at 4.8 TB/s (8 experts of 262 slots, W [1536, 512]: 31 us
-    against 41 directly; [3072, 4096]: 170 against 99)."""
-    tiles = min(rows, rows // 128 + E) * -(-K // 128)
-    return tiles <= 512 and 4 * E * N * K / 4.8e6 < 2 + 9e-3 * N
+def _transpose_first(E: int, N: int, K: int, plan: RoutingPlan) -> bool:
+    """Whether the input gradient is faster from transposed weights, as the
+    library that chooses the tiles says."""
+    return bool(lib().et_expert_input_grad_transposes_impl(E, N, K, plan.rows, plan.num_tokens, 0))
 
 
 def expert_gemm_input_grad(dc: torch.Tensor, w: torch.Tensor, plan: RoutingPlan, *, gather: bool = False,
@@ -545,7 +540,7 @@ def expert_gemm_input_grad(dc: torch.Tensor, w: torch.Tensor, plan: RoutingPlan,
     _require(w, "w", torch.bfloat16, 3)
     _check_plan(plan, w.device)
     E, N, K = w.shape
-    if wt is not None or _transpose_first(E, N, K, plan.rows):
+    if wt is not None or _transpose_first(E, N, K, plan):
         wt = expert_weight_transpose(w, plan, out=wt)
         return expert_gemm(dc, wt, plan, gather=gather, epilogue=epilogue, row_scale=row_scale, out=out)
     if E != plan.num_experts:

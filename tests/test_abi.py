@@ -321,3 +321,16 @@ def test_expert_gemm_route_does_not_read_the_capacitys_divisors(et):
     for mean in (40, 100, 200, 300, 500, 600):
         for exact in (0, 1):
             assert route(64 * mean - 1, exact) == route(64 * mean, exact), (mean, exact)
+
+
+@pytest.mark.parametrize("E,K,N,capacity,tokens,transposed", [
+    # us, through transposed weights / directly: 32 / 42, 42 / 50, 70 / 90, 79 / 149
+    (8, 1536, 512, 8 * 262, MANY, True), (8, 2048, 1536, 8 * 8, MANY, True), (8, 4096, 1536, 8 * 64, MANY, True),
+    (8, 7168, 512, 8 * 262, MANY, True), (24, 1536, 512, 24 * 8, MANY, True),
+    # 32 / 23, 55 / 43, 31 / 23, 171 / 83, 64 / 23: more than a round of thin tiles, or costly to transpose
+    (8, 512, 1536, 8 * 262, MANY, False), (24, 1536, 512, 24 * 262, MANY, False), (24, 512, 512, 24 * 262, MANY, False),
+    (8, 3072, 4096, 8 * 262, MANY, False), (24, 512, 1536, 24 * 64, MANY, False),
+    (64, 3072, 2048, 131072, 16384, False), (128, 4096, 1536, 65536 * 128, 65536, False)])
+def test_input_grad_transposes_only_where_thin_tiles_win(et, E, K, N, capacity, tokens, transposed):
+    f = et.lib().et_expert_input_grad_transposes_impl
+    assert bool(f(E, K, N, capacity, tokens, 256)) == transposed

@@ -233,8 +233,8 @@ int et_threshold_update(const float* logits, float* thr, int64_t num_tokens, int
  * `stream`.  Where et_route takes its pair lists (up to 256 experts), the
  * update's small passes run in the routing's launches (histogram; count with
  * the bin select; scan with the collect pass; place with the final select):
- * four launches for the two calls' seven (five below 32768 tokens; one for up
- * to 256 tokens, 16384 scores and 128 experts).
+ * four launches for the two calls' seven (five below 32768 tokens; one for small
+ * batches: up to 256 tokens with 64 experts, 200 with 80, 128 with 96, 32 with 128).
  * Workspaces: route_workspace as et_route's, thr_workspace as
  * et_threshold_update's; their byte ranges must not overlap
  * (ET_ERR_INVALID_ARGUMENT).

@@ -1345,18 +1345,22 @@ static int pairs_place(int64_t T, int64_t E, int32_t* counts, int32_t* expert_of
 // in its column of scores by fixing the key's bits from the top.  The rules,
 // the operations and so the bits are the other kernels'.  One CU reads the
 // logits and does every sigmoid, so it is taken for up to 256 tokens and 16384
-// scores; the statistic costs a wave 2.9 us per expert, so with the update for
-// up to 128 experts.  Measured (us on the device, this against the launches it
-// takes the place of): routing 8 tokens x 128 experts 3.6 / 13.2, 128 x 64 7.7 /
-// 11.2, 256 x 32 10.0 / 10.6, 512 x 32 17.5 / 10.6 (left to those); routing with
-// update 61 x 8 6.1 / 23, 128 x 64 19 / 24, 61 x 128 30 / 27 (and 20 us less on
-// the host), 61 x 256 58 / 38 (left to those).
+// scores.  Measured (us on the device, this against the launches it takes the
+// place of): 8 tokens x 128 experts 4.6 / 13.1, 128 x 64 8.4 / 11.7, 256 x 32 11.2 /
+// 11.9, 200 x 80 15.4 / 13.9 (an eager call of the last 15.6 against 25, two launches
+// less on the host), 512 x 32 17.5 / 10.6 (left to those).
+// The statistic costs a wave 2.9 us per expert, and more with the tokens, so with
+// the update the line lies where one block takes 28 us (route_update_is_small): up to
+// there an eager call is faster (8 x 128 26.8 us a call / 30.4 with the five launches,
+// bound by their host time; 61 x 96 24 / 30; 128 x 96 28.2 / 31.4; 200 x 80 28.5 / 32.9;
+// past it 61 x 128 30.2 / 30.6, 100 x 128 33.5 / 30.6), though in a graph the launches
+// alone take 24 to 27 above about 20 us: 32 x 64 16.4 / 23.7, 61 x 96 24.8 / 26.7, 128 x
+// 80 25.4 / 26.5, 8 x 128 27.3 / 23.6, 128 x 96 28.8 / 26.7, 100 x 128 34.1 / 26.4.
 constexpr int kSmallWaves = 16;
 constexpr int kSmallThreads = kSmallWaves * kWave;
 constexpr int kSmallEntries = 16384;      // T * (E | 1) scores in LDS (64 KiB)
 constexpr int kSmallTokens = 256;
 constexpr int kSmallExperts = 256;
-constexpr int kSmallUpdateExperts = 128;
 
 struct SmallUpdate {
     float* thr;        // [E], rewritten
@@ -1616,7 +1620,10 @@ int route_update_place_final(int64_t T, int64_t E, int32_t* counts, int32_t* exp
     return check_launch("route_place_kernel (with the final select)");
 }
 
-bool route_update_is_small(int64_t T, int64_t E) { return route_is_small(T, E) && E <= kSmallUpdateExperts; }
+bool route_update_is_small(int64_t T, int64_t E)
+{
+    return route_is_small(T, E) && E <= (T <= 32 ? 128 : T <= 64 ? 112 : T <= 128 ? 96 : 80);
+}
 
 int route_update_small(const float* logits, float* thr, int64_t T, int64_t E, int32_t* counts,
                        int32_t* expert_offsets, int32_t* token_offsets, int32_t* sorted_token, float* slot_gate,
@@ -1858,3 +1865,6 @@ extern "C" int et_copy_slots_impl(const int32_t* sorted_token, const float* slot
         c, n, (bits & 15) == 0);
     return check_launch("copy_slots_kernel");
 }
+
+// Whether routing with the EMA update of such a batch takes one block (for tests).
+extern "C" int et_route_update_is_small_impl(int64_t T, int64_t E) { return route_update_is_small(T, E) ? 1 : 0; }

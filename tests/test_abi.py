@@ -334,3 +334,12 @@ def test_expert_gemm_route_does_not_read_the_capacitys_divisors(et):
 def test_input_grad_transposes_only_where_thin_tiles_win(et, E, K, N, capacity, tokens, transposed):
     f = et.lib().et_expert_input_grad_transposes_impl
     assert bool(f(E, K, N, capacity, tokens, 256)) == transposed
+
+
+@pytest.mark.parametrize("T,E,small", [(8, 64, 1), (8, 128, 1), (32, 128, 1), (61, 112, 1), (128, 96, 1), (200, 80, 1),
+                                       (256, 63, 1), (250, 65, 1), (8, 129, 0),
+                                       (61, 128, 0), (100, 128, 0), (100, 112, 0), (128, 127, 0), (128, 97, 0)])
+def test_one_block_routing_with_update_only_where_it_is_no_slower(et, T, E, small):
+    """In a call of its own: past the line one block takes longer than the five
+    launches' host time."""
+    assert et.lib().et_route_update_is_small_impl(T, E) == small

@@ -27,7 +27,8 @@ def _batch(T, E, seed):
 
 @pytest.mark.parametrize("T,E", [(1, 1), (1, 256), (15, 8), (17, 64), (16, 65), (63, 256), (64, 256), (127, 129),
                                  (128, 127), (128, 128), (252, 65), (253, 65), (256, 63), (256, 64), (255, 8),
-                                 (256, 1), (257, 8), (64, 300)])
+                                 (256, 1), (257, 8), (64, 300), (32, 128), (33, 128), (64, 112), (64, 113), (65, 112),
+                                 (128, 96), (128, 97), (129, 80), (129, 81)])
 def test_small_routing_and_update_equal_the_oracle(et, orc, dev, T, E):
     print(f"small route T={T} E={E}", flush=True)
     for seed in (0, 1):

@@ -71,6 +71,7 @@ _SIGNATURES = {
     "et_expert_gemm_route_impl": (_int, [_int, _int, _int, _i64, _i64, _i64, _i64, _int, _i64, _int]),
     "et_expert_input_grad_transposes_impl": (_int, [_i64, _i64, _i64, _i64, _i64, _int]),
     "et_route_update_is_small_impl": (_int, [_i64, _i64]),
+    "et_router_small_tile_impl": (_int, [_i64, _i64, _i64]),
     "et_copy_slots_impl": (_int, [_p, _p, _p, _i64, _p, _p, _p, _p]),
     "et_expert_input_grad_impl": (_int, [_p, _i64, _p, _p, _p, _i64, _i64, _i64, _i64, _int, _p, _p, _p]),
     "et_expert_weight_transpose": (_int, [_p, _p, _i64, _i64, _i64, _i64, _p, _p]),

@@ -498,8 +498,25 @@ __global__ __launch_bounds__(MW * kWave) void router_logits_kernel(
 // twice as long), and the tiled kernel where none does.  Measured (us, this
 // against the tiled kernel): 128 experts, d = 4096: 8 tokens 8.0 / 34, 512 9.6 /
 // 35, 1024 13.3 / 35, 4096 24.9 / 36 (8192: 46 / 37, left to the tiled one); 64
-// experts, d = 2048: 8 tokens 5.1 / 12.6, 4096 9.7 / 13.2, 8192 14.2 / 14.0.
+// experts, d = 2048: 8 tokens 5.1 / 12.6, 4096 10.5 / 14.3, 8192 14.6 / 14.7.  Over half
+// of the CUs with full tiles of 32 x 64 (49 to 64 experts, over 4096 tokens) the
+// load path loses to the tiled kernel's once rows are long: 6000 tokens, 64 experts,
+// d = 1024 9.1 / 9.4, 4096 24.9 / 24.0, 7168 40.9 / 38.3; 48 experts, d = 7168 35.9 / 37.7.
 constexpr int64_t kRouterSmallWaves = 256;
+constexpr int kRouterSmallFullExperts = 56;    // (with one group of up to 64 experts)
+constexpr int kRouterSmallLongRow = 2048;
+
+// The wave tile: 1 to 4 for 16 x 16, 16 x 32, 32 x 32 and 32 x 64; 0: the tiled kernel.
+int router_small_tile(int64_t T, int64_t d, int64_t E)
+{
+    const auto waves = [&](int64_t t, int64_t e) { return ((T + t - 1) / t) * ((E + e - 1) / e); };
+    if (waves(16, 16) <= kRouterSmallWaves) return 1;
+    if (waves(16, 32) <= kRouterSmallWaves) return 2;
+    if (waves(32, 32) <= kRouterSmallWaves) return 3;
+    if (waves(32, 64) > kRouterSmallWaves) return 0;
+    const bool slow = E > kRouterSmallFullExperts && E <= 64 && d > kRouterSmallLongRow;
+    return slow && waves(32, 64) > kRouterSmallWaves / 2 ? 0 : 4;
+}
 
 template <int MX, int ME, int U>
 __global__ __launch_bounds__(kWave) void router_logits_small_kernel(const uint16_t* __restrict__ x,
@@ -663,15 +680,18 @@ extern "C" int et_router_logits(const void* x, const void* w, int64_t T, int64_t
     const uint16_t* xp = static_cast<const uint16_t*>(x);
     const uint16_t* wp = static_cast<const uint16_t*>(w);
     // few tokens: the smallest wave tile that leaves a CU to each wave
-    auto small = [&](auto kernel, int mx, int me) {
+    const auto small = [&](auto kernel, int mx, int me) {
         const int64_t waves = ((T + 16 * mx - 1) / (16 * mx)) * ((E + 16 * me - 1) / (16 * me));
-        if (waves > kRouterSmallWaves) return false;
         kernel<<<dim3((unsigned)waves), dim3(kWave), 0, s>>>(xp, wp, (int)T, (int)d, (int)E, logits);
-        return true;
-    };
-    if (small(router_logits_small_kernel<1, 1, 16>, 1, 1) || small(router_logits_small_kernel<1, 2, 12>, 1, 2) ||
-        small(router_logits_small_kernel<2, 2, 8>, 2, 2) || small(router_logits_small_kernel<2, 4, 8>, 2, 4))
         return check_launch("router_logits_small_kernel");
+    };
+    switch (router_small_tile(T, d, E)) {
+        case 1: return small(router_logits_small_kernel<1, 1, 16>, 1, 1);
+        case 2: return small(router_logits_small_kernel<1, 2, 12>, 1, 2);
+        case 3: return small(router_logits_small_kernel<2, 2, 8>, 2, 2);
+        case 4: return small(router_logits_small_kernel<2, 4, 8>, 2, 4);
+        default: break;
+    }
     const RouterLaunch L = router_launch(T);
     const int64_t ntiles = (T + 32 * L.mw * L.mt - 1) / (32 * L.mw * L.mt);
     const dim3 grid((unsigned)std::min<int64_t>(ntiles, kRouterMaxBlocks));
@@ -780,3 +800,6 @@ extern "C" int et_router_route(const void* x, const void* w, const float* thr, i
                                    expert_offsets, token_offsets, sorted_token, slot_gate, token_slot, slot_capacity,
                                    s);
 }
+
+// The kernel of such a router_logits call (for tests): see router_small_tile.
+extern "C" int et_router_small_tile_impl(int64_t T, int64_t d, int64_t E) { return router_small_tile(T, d, E); }

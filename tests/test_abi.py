@@ -343,3 +343,13 @@ def test_one_block_routing_with_update_only_where_it_is_no_slower(et, T, E, smal
     """In a call of its own: past the line one block takes longer than the five
     launches' host time."""
     assert et.lib().et_route_update_is_small_impl(T, E) == small
+
+
+@pytest.mark.parametrize("T,d,E,tile", [
+    (1, 8, 1, 1), (4096, 7168, 16, 1), (512, 4096, 128, 1), (1024, 4096, 128, 2), (2048, 4096, 128, 3),
+    (4096, 7168, 128, 4), (4097, 4096, 128, 0),
+    (4096, 7168, 64, 3), (4097, 2048, 64, 4), (8192, 1024, 64, 4), (8193, 1024, 64, 0),
+    # long rows of 64 experts: the tiled kernel is 3 to 7% faster
+    (4097, 4096, 64, 0), (6000, 7168, 64, 0), (8192, 2056, 57, 0), (8192, 7168, 48, 4)])
+def test_router_logits_tile(et, T, d, E, tile):
+    assert et.lib().et_router_small_tile_impl(T, d, E) == tile

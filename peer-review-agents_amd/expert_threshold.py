@@ -22,7 +22,7 @@ dXp) have one row per slot.
 """
 from __future__ import annotations
 
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 from typing import Optional
 
 import torch
@@ -140,6 +140,20 @@ class RoutingPlan:
     def device(self) -> torch.device:
         return self.token_offsets.device
 
+    def __getstate__(self) -> dict:
+        """The fields, the slot arrays at their own size: those of a small plan are
+        views into buffers of the capacity (see _shrink), which a pickle or a
+        torch.save would write whole, unset entries and all."""
+        state = dict(self.__dict__)
+        for name in ("sorted_token", "slot_gate", "token_slot"):
+            t = state[name]
+            if t.untyped_storage().nbytes() > t.numel() * t.element_size():
+                state[name] = t.clone()
+        return state
+
+    def __copy__(self) -> "RoutingPlan":
+        return replace(self)
+
 
 def route_workspace_bytes(num_tokens: int, num_experts: int) -> int:
     return int(lib().et_route_workspace_bytes(num_tokens, num_experts))
@@ -197,8 +211,8 @@ def _shrink(plan: RoutingPlan, S: int) -> None:
     Where the capacity is large they become exactly-sized copies, so the T*E
     buffers are released (a plan held until a backward pass then pins 12 bytes
     per slot, not per token-expert pair); small ones (256 KiB an array at most)
-    are views, which spares a small call three copies (8 us on the device, 14
-    on the host)."""
+    are views, which spares a small call the copy's launch and three
+    allocations (a pickled plan has them at their own size)."""
     plan.num_slots = S
     if plan.capacity <= _KEEP_ENTRIES:
         plan.sorted_token = plan.sorted_token[:S]

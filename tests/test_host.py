@@ -82,3 +82,29 @@ def test_expert_gemm_fp8_checks_shapes_like_bf16(et):
             call(n=72, epilogue="swiglu")
         with pytest.raises(ValueError, match="slot-major"):
             call(a_rows=99, gather=False)
+
+
+def _small_plan(et, S=5, cap=4096):
+    """A plan as a small batch's routing leaves it: slot arrays of S entries, views
+    into buffers of the capacity."""
+    i32 = torch.int32
+    whole = [torch.full((cap,), 77, dtype=i32), torch.full((cap,), 0.5), torch.full((cap,), 99, dtype=i32)]
+    return et.RoutingPlan(torch.tensor([2, 3], dtype=i32), torch.tensor([0, 2, 5], dtype=i32),
+                          torch.arange(S + 1, dtype=i32), *(t[:S] for t in whole), S, 2, S, S)
+
+
+def test_a_saved_plan_holds_its_slots_and_not_the_capacity(et, tmp_path):
+    import copy
+    import pickle
+    plan = _small_plan(et)
+    torch.save(plan, tmp_path / "plan.pt")
+    loaded = [torch.load(tmp_path / "plan.pt", weights_only=False), pickle.loads(pickle.dumps(plan)), copy.deepcopy(plan)]
+    for other in loaded:
+        for name in ("sorted_token", "slot_gate", "token_slot", "counts", "expert_offsets", "token_offsets"):
+            a, b = getattr(plan, name), getattr(other, name)
+            assert torch.equal(a, b) and a.dtype == b.dtype
+            assert b.untyped_storage().nbytes() == b.numel() * b.element_size(), name
+        assert (other.num_tokens, other.num_experts, other.capacity, other.num_slots) == (5, 2, 5, 5)
+    assert (tmp_path / "plan.pt").stat().st_size < 8192
+    shallow = copy.copy(plan)
+    assert shallow is not plan and shallow.sorted_token is plan.sorted_token

@@ -1044,22 +1044,23 @@ extern "C" int et_expert_input_grad_impl(const void* dc, int64_t dc_rows, const 
 
 // Whether the input gradient (a sum of K, N columns) is faster through transposed
 // weights: the thin tiles need them, which win where at most one round of them is
-// there.  256-row tiles on the weights as they are then take one round, 9.5 + 19.7 K
-// / 1000 us, the thin ones their share of 9.3 + 16.7 K / 1000, and the transpose moves
-// the weights twice at 6.3 TB/s, 4.5 us beside (6 at least) and 4 until the thin
-// tiles stream.  Measured (us, transposed against directly): 8 experts of 262 slots, K =
-// 1536, N = 512 32 / 42, K = 2048, N = 1536 42 / 50 (8 slots each), K = 512, N = 1536
-// 32 / 23, K = 3072, N = 4096 171 / 83; 24 of 8 slots, K = 1536, N = 512 35 / 41; 24 of
-// 262, 292 thin tiles, 55 / 43.
+// there (short sums: five eighths of one).  256-row tiles on the weights as they are
+// then take one round, 9.5 + 19.7 K / 1000 us and up to 2.5 by their slots; the thin
+// ones their share of 9.3 + 16.7 K / 1000, and the transpose moves the weights twice at
+// 6.3 TB/s, 4.5 us beside (6 at least) and 4 until the thin tiles stream.  Measured
+// (us, transposed / directly): 8 experts of 262 slots, K = 512, N = 512 17 / 22, K =
+// 1536, N = 512 32 / 42, K = 512, N = 1536 32 / 23, K = 3072, N = 4096 171 / 83; of 8
+// slots, K = 2048, N = 1536 42 / 50; 24 of 8 slots, K = 1536, N = 512 35 / 41; 24 of 262
+// slots (292 thin tiles) 55 / 43.
 static bool input_grad_transposes(int64_t E, int64_t K, int64_t N, int64_t capacity, int64_t tokens, int cus)
 {
     const TileCall c{(int)K, cus, false, false, false};
     const int64_t nt = (N + 127) / 128, most = std::min(tokens, capacity);
     const int64_t tiles_max =
         std::min(capacity / kThinTile + E, E * std::min((most + kThinTile - 1) / kThinTile, capacity)) * nt;
-    if (tiles_max > cus) return false;
-    const int64_t mean = std::min<int64_t>((capacity + E - 1) / E, kThinTile);
-    const int64_t direct = 9500 + 197 * K / 10, other = 9300 + 167 * K / 10;
+    if (tiles_max > (K < 1024 ? 5 * (int64_t)cus / 8 : cus)) return false;
+    const int64_t slots = (capacity + E - 1) / E, mean = std::min<int64_t>(slots, kThinTile);
+    const int64_t direct = 9500 + 197 * K / 10 + 10 * std::min<int64_t>(slots, kBM), other = 9300 + 167 * K / 10;
     const int64_t transpose = std::max<int64_t>(6000, 4500 + E * K * N * 4 / 6300) + 4000;
     return transpose + other * thin_share(c, (int)mean, (int)tiles_max) / 1000 < direct;
 }

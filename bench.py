@@ -357,8 +357,9 @@ def expert_gemm_leg(et, dev, stream, plan, X, reps: int = 3) -> dict:
     fl_up, fl_down = 2.0 * S * d * 2 * F, 2.0 * S * F * d
     # backward: the down projection's input gradient fused with the combine
     # backward (dY gathered, rows times the slot gate), the gate/up
-    # projection's input gradient (both through the transposed weights of the
-    # experts with slots), and both weight gradients (f32)
+    # projection's input gradient (both on the weights as they are, the default
+    # form, and through the transposed weights of the experts with slots, the
+    # wt= form), and both weight gradients (f32)
     dy = torch.randn(T, d, device=dev, generator=g).to(torch.bfloat16)
     dgu = torch.randn(S, 2 * F, device=dev, generator=g).to(torch.bfloat16)
     w2t = torch.empty(E, F, d, dtype=torch.bfloat16, device=dev)
@@ -366,9 +367,12 @@ def expert_gemm_leg(et, dev, stream, plan, X, reps: int = 3) -> dict:
     dh = torch.empty(S, F, dtype=torch.bfloat16, device=dev)
     dxp = torch.empty(S, d, dtype=torch.bfloat16, device=dev)
     t_tr2 = timed(lambda: et.expert_weight_transpose(w2, plan, out=w2t))
-    t_down_bwd = timed(lambda: et.expert_gemm_input_grad(dy, w2, plan, gather=True, row_scale=plan.slot_gate,
-                                                          wt=w2t, out=dh))
-    t_up_bwd = timed(lambda: et.expert_gemm_input_grad(dgu, w1, plan, wt=w1t, out=dxp))
+    def down_bwd(**kw):
+        return et.expert_gemm_input_grad(dy, w2, plan, gather=True, row_scale=plan.slot_gate, out=dh, **kw)
+
+    t_down_bwd, t_down_bwd_tr = timed(down_bwd), timed(lambda: down_bwd(wt=w2t))
+    t_up_bwd = timed(lambda: et.expert_gemm_input_grad(dgu, w1, plan, out=dxp))
+    t_up_bwd_tr = timed(lambda: et.expert_gemm_input_grad(dgu, w1, plan, wt=w1t, out=dxp))
     # the activation for training, on the kept gate/up output h (HBM-bound:
     # 6F bytes per slot forward, 10F backward)
     hs = torch.empty(S, F, dtype=torch.bfloat16, device=dev)
@@ -414,6 +418,8 @@ def expert_gemm_leg(et, dev, stream, plan, X, reps: int = 3) -> dict:
             "backward": {"weight_transpose_down_ms": round(t_tr2, 3),
                          "down_input_grad_fused_combine_bwd_ms": round(t_down_bwd, 3),
                          "gate_up_input_grad_ms": round(t_up_bwd, 3),
+                         "down_input_grad_through_transpose_ms": round(t_down_bwd_tr, 3),
+                         "gate_up_input_grad_through_transpose_ms": round(t_up_bwd_tr, 3),
                          "gate_up_weight_grad_ms": round(t_wg_up, 3),
                          "gate_up_weight_grad_TFLOP/s": round(fl_wg_up / (t_wg_up * 1e-3) / 1e12, 1),
                          "down_weight_grad_ms": round(t_wg_down, 3),

@@ -812,8 +812,10 @@ enum GemmRoute { kRouteThin = 0, kRouteBig = 1, kRouteDevice = 2 };
 
 // On the device (kRouteDevice) both kernels are launched and decide from the
 // slot counts (expert_gemm_split); the one that finds no work takes 4 to 5 us, a
-// fifth of the shortest calls.  So that is for calls of about 50 us and more and
-// for those where thin tiles may gain more than it costs; the others go to
+// fifth of the shortest calls.  So that is for calls of about 50 us and more, and
+// for shorter ones where thin tiles may gain more than it costs (4.5 us with SwiGLU: 1.1
+// to 1.35 times there; 10 us for plain ones: at 4.5 1.05 at even loads and 0.91 at Zipf's);
+// the others go to
 //   - the thin kernel where no split of the slots makes it slower: its tiles
 //     are few at their most, or no expert has more slots than one of its tiles
 //     and every count of busy experts is within 3%; also just above one round at
@@ -845,20 +847,25 @@ GemmRoute expert_gemm_route(const TileCall& c, int64_t E, int64_t N, int64_t cap
     const int64_t likely = exact || tokens > capacity ? most : std::max<int64_t>(1, tokens / 4);
     if (most <= kThinTile) {
         const int64_t all = std::min(E, capacity);
-        const auto at = [&](int64_t busy) { return ratio(busy * nt, busy, std::min(likely, (capacity + busy - 1) / busy)); };
-        int64_t lo = at(all), hi = lo;
+        // (at the mean slots of the busy experts, and for the worst case, with three
+        // quarters of the experts or more busy, at three times these: an uneven load's
+        // heavy ones)
+        const auto at = [&](int64_t busy, int64_t times) {
+            return ratio(busy * nt, busy, std::min(most, times * std::min(likely, (capacity + busy - 1) / busy)));
+        };
+        int64_t lo = at(all, 1), hi = at(all, 3);
         for (int64_t r = 1; r <= 4; ++r)   // (both sides of each of the first rounds' ends)
             for (int64_t busy = r * c.cus / nt; busy <= r * c.cus / nt + 1; ++busy)
                 if (busy >= 1 && busy < all) {
-                    lo = std::min(lo, at(busy));
-                    hi = std::max(hi, at(busy));
+                    lo = std::min(lo, at(busy, 1));
+                    hi = std::max(hi, at(busy, 4 * busy >= 3 * all ? 3 : 1));
                 }
         if (hi <= 1030) return kRouteThin;
         if (lo >= 970) return kRouteBig;
         if (big_us(all * nb) >= kDeviceUs) return kRouteDevice;
-        return at(all) <= 1000 ? kRouteThin : kRouteBig;
+        return at(all, 1) <= 1000 ? kRouteThin : kRouteBig;
     }
-    const int64_t mean = exact ? (capacity + E - 1) / E : std::min<int64_t>(likely, kThinTile / 2);
+    const int64_t mean = exact ? (capacity + E - 1) / E : std::min<int64_t>(likely, kThinTile);
     // slot tiles at most, and at a likely load
     const int64_t tiles_max =
         std::min(capacity / kThinTile + E, E * std::min((most + kThinTile - 1) / kThinTile, capacity)) * nt;
@@ -879,7 +886,7 @@ GemmRoute expert_gemm_route(const TileCall& c, int64_t E, int64_t N, int64_t cap
     if (big_us(E * nb) >= kDeviceUs) return kRouteDevice;
     // (an eighth more tiles, for an uneven load)
     if (exact && ratio(tiles * 9 / 8, E, mean) <= 950) return kRouteThin;
-    return (1000 - even) * big_us(E * nb) >= 4500 ? kRouteDevice : kRouteBig;
+    return (1000 - even) * big_us(E * nb) >= (c.swiglu ? 4500 : 10000) ? kRouteDevice : kRouteBig;
 }
 
 // Argument checks and launch of the entry points (es = bytes per operand

@@ -110,7 +110,7 @@ __host__ __device__ inline int thin_share(const TileCall& c, int n, int tiles)
     }
     int share = of(445, c.K > 4096 ? 510 : 480, 515, 535);
     if (c.swiglu) share -= share * 150 / (c.K + 150);   // (the 256-row epilogue)
-    if (c.K > 2048 && tiles > c.cus && tiles <= 3 * c.cus) share += n <= (c.K <= 4096 ? 32 : 16) ? 60 : c.K <= 4096 ? 100 : 130;
+    if (c.K > 2048 && tiles > c.cus && tiles <= 3 * c.cus) share += n <= (c.K <= 5120 ? 32 : 16) ? 60 : c.K <= 5120 ? 100 : 130;
     return share;
 }
 
@@ -130,13 +130,14 @@ __host__ __device__ inline int thin_time(const TileCall& c, int tiles, int share
     return (tiles + c.cus - 1) / c.cus * (thin_few(c, tiles) && share > 950 ? 950 : share);
 }
 
-// `tiles` 256-row tiles in a call of `thin` thin ones.  (At K = 4096 a full round
-// of bf16 weights is bound by HBM: 1.3 times a partial one's time.)
+// `tiles` 256-row tiles in a call of `thin` thin ones.  (From K = 4096 on a full
+// round of bf16 weights is bound by HBM: 1.3 times a partial one's time, of which the
+// thin kernel pays some too above 5120.)
 __host__ __device__ inline int big_time(const TileCall& c, int tiles, int thin)
 {
     const int t = (tiles + c.cus - 1) / c.cus * 1000;
-    if (c.fp8 || c.K <= 2048 || c.K > 4096 || thin > 3 * c.cus) return t;
-    const int hbm = 1300 * tiles / c.cus;
+    if (c.fp8 || c.K <= 2048 || thin > 3 * c.cus) return t;
+    const int hbm = (c.K <= 5120 ? 1300 : 1100) * tiles / c.cus;
     return t > hbm ? t : hbm;
 }
 
